@@ -3,8 +3,9 @@
 // by 1/sqrt(head_dim), softmax, weighted value mix), as split-K flash
 // decoding:
 //
-//   attn_kernel (f32 K/V; BF16 K/V decode runs on the matrix cores,
-//   attn_dec_mfma_kernel below): grid (splits, kv_heads, rows); block = 256
+//   attn_kernel (f32 K/V decode; BF16 K/V decode runs on the matrix cores,
+//   attn_dec_mfma_kernel below, and chunked prefill on attn_prefill_kernel or
+//   attn_prefill_f32_kernel): grid (splits, kv_heads, rows); block = 256
 //   threads.
 //   Each block owns one KV head, one query row and one contiguous slice of
 //   that row's visible positions [0, pos]; it streams the slice in tiles of
@@ -736,6 +737,39 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf16x8 &hi, bf16x8 &
 // stays one aligned 16-byte read.
 __device__ __forceinline__ int vcol(int d, int p) { return (((p >> 3) ^ ((d >> 3) & 7)) << 3) | (p & 7); }
 
+// A prefill lane's results, O^T registers of its M row: dims
+// 32 u + 8 (r / 4) + 4 half + r % 4. One split: the normalised output at
+// element ob (with its BF16 halves where asked for); more: the partial.
+template <int HD>
+__device__ __forceinline__ void store_prefill_rows(const AttnArgs &a, const f32x16 (&oacc)[HD / 32], float m2, float l,
+                                                   float *part, size_t ob, int S, int half) {
+    constexpr int UT = HD / 32;
+    if (S == 1) {
+        const float inv = 1.0f / l;
+        float *o = a.out + ob;
+#pragma unroll
+        for (int u = 0; u < UT; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 v = f32x4{oacc[u][4 * q] * inv, oacc[u][4 * q + 1] * inv, oacc[u][4 * q + 2] * inv,
+                                      oacc[u][4 * q + 3] * inv};
+                *(f32x4 *)(o + 32 * u + 8 * q + 4 * half) = v;
+                if (a.out_hi) store_halves4(a.out_hi, a.out_lo, ob + 32 * u + 8 * q + 4 * half, v);
+            }
+    } else {
+#pragma unroll
+        for (int u = 0; u < UT; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *(f32x4 *)(part + 32 * u + 8 * q + 4 * half) =
+                    f32x4{oacc[u][4 * q], oacc[u][4 * q + 1], oacc[u][4 * q + 2], oacc[u][4 * q + 3]};
+        if (half == 0) {
+            part[HD] = m2;
+            part[HD + 1] = l;
+        }
+    }
+}
+
 template <int HD, int G>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill_kernel(AttnArgs a, int rows, int S, int span) {
     constexpr int RW = 32 / G, MV = RW * G;
@@ -914,32 +948,245 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         b ^= 1;
     }
     if (!rvalid) return;
-    // O^T registers: lane's M row, dims 32 u + 8 (r / 4) + 4 half + r % 4.
-    if (S == 1) {
-        const float inv = 1.0f / l;
-        const size_t ob = (size_t)row * (size_t)a.q_heads * HD + (size_t)head * HD;
-        float *o = a.out + ob;
+    store_prefill_rows<HD>(a, oacc, m2, l, part, (size_t)row * a.q_heads * HD + (size_t)head * HD, S, half);
+}
+
+// ---------------------------------------------------------------------------
+// Chunked prefill over an f32 K/V cache on the matrix cores: the flash
+// attention of attn_prefill_kernel (same blocks, rows per wave, LDS row
+// permutation, transposed V, delayed rescaling and split partials) with every
+// f32 operand as three BF16 parts (hi = the top 16 bits, mid = bf16 of the
+// rest, lo = what is left: all 24 bits exactly). Of the nine part products
+// the six above 2^-24 are taken, smallest first; the score's small ones add up
+// in an accumulator of their own.
+//
+// Bound: the matrix cores (six BF16 products per f32 one, i.e. at most 1/6 of
+// the BF16 rate; the f32 MFMA's rate is 1/16 of it). K/V are split once per
+// block and tile while they are staged (64 keys x head_dim, three planes of K
+// rows and of V columns in LDS: 102 KB at head_dim 128, so one block of four
+// waves per CU with 512 registers each; the next tile's rows wait in
+// registers during the products).
+// Measured on 512-row chunks of a 1,500-token prompt, 32 q / 8 KV heads of
+// 128: 40 / 80 / 128 us a chunk against 1,025 to 1,781 us on the vector ALUs
+// (attn_kernel, which decodes only now); that prompt through two Q4 layers of
+// the shape 11.94 -> 4.36 ms, its logits no further from 64-bit ones.
+// ---------------------------------------------------------------------------
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+
+struct Parts2 {  // two values' parts, packed
+    uint32_t h, m, l;
+};
+__device__ __forceinline__ Parts2 split3(float a, float b) {
+    const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+    const float ra = a - __uint_as_float(ua & 0xFFFF0000u), rb = b - __uint_as_float(ub & 0xFFFF0000u);
+    const __bf16 ma = (__bf16)ra, mb = (__bf16)rb;
+    const __bf16 la = (__bf16)(ra - (float)ma), lb = (__bf16)(rb - (float)mb);
+    Parts2 p;
+    p.h = __builtin_amdgcn_perm(ub, ua, 0x07060302u);
+    p.m = (uint32_t)__builtin_bit_cast(uint16_t, ma) | ((uint32_t)__builtin_bit_cast(uint16_t, mb) << 16);
+    p.l = (uint32_t)__builtin_bit_cast(uint16_t, la) | ((uint32_t)__builtin_bit_cast(uint16_t, lb) << 16);
+    return p;
+}
+// Eight values' parts as three matrix operands.
+__device__ __forceinline__ void split3x8(const float (&v)[8], bf16x8 (&out)[3]) {
+    u32x4 w[3];
 #pragma unroll
-        for (int u = 0; u < UT; ++u)
+    for (int i = 0; i < 4; ++i) {
+        const Parts2 p = split3(v[2 * i], v[2 * i + 1]);
+        w[0][i] = p.h;
+        w[1][i] = p.m;
+        w[2][i] = p.l;
+    }
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const f32x4 v = f32x4{oacc[u][4 * q] * inv, oacc[u][4 * q + 1] * inv, oacc[u][4 * q + 2] * inv,
-                                      oacc[u][4 * q + 3] * inv};
-                *(f32x4 *)(o + 32 * u + 8 * q + 4 * half) = v;
-                if (a.out_hi) store_halves4(a.out_hi, a.out_lo, ob + 32 * u + 8 * q + 4 * half, v);
+    for (int k = 0; k < 3; ++k) out[k] = __builtin_bit_cast(bf16x8, w[k]);
+}
+
+constexpr int kF32LdV = 64 + 8;  // transposed V row: 64 positions + 16 bytes
+template <int HD>
+constexpr size_t prefill_f32_lds_bytes() { return (size_t)3 * 2 * (64 * HD + HD * kF32LdV); }
+
+template <int HD, int G>
+__global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_kernel(AttnArgs a, int rows, int S,
+                                                                                     int span) {
+    constexpr int RW = 32 / G, MV = RW * G;
+    constexpr int LDV = kF32LdV;
+    constexpr int KSTEPS = HD / 16, UT = HD / 32;
+    constexpr int CPR = HD / 8;    // 16-byte chunks per K row and plane
+    constexpr int KU = HD / 32;    // K staging units (8 dims of a row) per thread
+    constexpr int VU = HD / 64;    // V staging units (4 positions x 4 dims) per thread
+    extern __shared__ __attribute__((aligned(16))) uint16_t smem_f32[];
+    uint16_t *ks = smem_f32;               // [3][64][HD], chunks swizzled as in attn_prefill_kernel
+    uint16_t *vt = smem_f32 + 3 * 64 * HD;  // [3][HD][LDV]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n = lane & 31, half = lane >> 5;
+    const int rb = blockIdx.x, g = blockIdx.y, split = blockIdx.z;
+    const int row = rb * 4 * RW + wave * RW + n / G;
+    const int head = g * G + n % G;
+    const bool rvalid = n < MV && row < rows;
+    const int off = (int)a.offset;
+    const int my_pos = off + row;
+    const int first_pos = off + rb * 4 * RW;
+    const int ctx = off + min(rows, (rb + 1) * 4 * RW);
+    const int start = split * span;
+    const int end = min(start + span, ctx);
+    float *part = a.part + (((size_t)row * a.q_heads + head) * S + split) * (HD + 2);
+    if (start >= ctx) {  // block-uniform: no row of this block reaches the split
+        if (rvalid && half == 0) part[HD] = -INFINITY;
+        return;
+    }
+
+    // The next tile's rows in registers. K unit: 8 dims of position idx / CPR;
+    // V unit: 4 dims of positions 4 (idx / (HD / 4)) .. + 3.
+    const float *kbase = (const float *)a.k, *vbase = (const float *)a.v;
+    f32x4 kr[KU][2], vr[VU][4];
+    auto fetch = [&](int t0) {
+        const int page = a.page_table[t0 / a.page_size];
+        const size_t tile = (((size_t)page * a.kv_heads + g) * a.page_size + (t0 % a.page_size)) * HD;
+#pragma unroll
+        for (int c = 0; c < KU; ++c) {
+            const int idx = tid + kThreads * c;
+            const float *src = kbase + tile + (size_t)(idx / CPR) * HD + (idx % CPR) * 8;
+            kr[c][0] = *(const f32x4 *)src;
+            kr[c][1] = *(const f32x4 *)(src + 4);
+        }
+#pragma unroll
+        for (int c = 0; c < VU; ++c) {
+            const int idx = tid + kThreads * c, p0 = 4 * (idx / (HD / 4)), d0 = 4 * (idx % (HD / 4));
+#pragma unroll
+            for (int i = 0; i < 4; ++i)  // positions past the split end may be unwritten: zeros (p = 0 there)
+                vr[c][i] = t0 + p0 + i < end ? *(const f32x4 *)(vbase + tile + (size_t)(p0 + i) * HD + d0)
+                                             : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int c = 0; c < KU; ++c) {
+            const int idx = tid + kThreads * c, r = krow_of(idx / CPR);
+            const float v[8] = {kr[c][0][0], kr[c][0][1], kr[c][0][2], kr[c][0][3],
+                                kr[c][1][0], kr[c][1][1], kr[c][1][2], kr[c][1][3]};
+            bf16x8 w[3];
+            split3x8(v, w);
+            uint16_t *dst = ks + r * HD + (((idx % CPR) ^ (r % CPR)) << 3);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) *(bf16x8 *)(dst + k * 64 * HD) = w[k];
+        }
+#pragma unroll
+        for (int c = 0; c < VU; ++c) {
+            const int idx = tid + kThreads * c, p0 = 4 * (idx / (HD / 4)), d0 = 4 * (idx % (HD / 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const Parts2 x = split3(vr[c][0][e], vr[c][1][e]), y = split3(vr[c][2][e], vr[c][3][e]);
+                uint16_t *dst = vt + (d0 + e) * LDV + vcol(d0 + e, p0);
+                *(u32x2_t *)dst = u32x2_t{x.h, y.h};
+                *(u32x2_t *)(dst + HD * LDV) = u32x2_t{x.m, y.m};
+                *(u32x2_t *)(dst + 2 * HD * LDV) = u32x2_t{x.l, y.l};
             }
-    } else {
+        }
+    };
+    fetch(start);
+
+    // Q^T operands, pre-scaled by log2(e) / sqrt(HD) (scores in the exp2 domain).
+    bf16x8 q3[KSTEPS][3];
+    {
+        const float sl2 = (1.0f / sqrtf((float)HD)) * 1.44269504088896340736f;
+        const float *qp = a.q + (size_t)(rvalid ? row : 0) * a.q_stride + (size_t)head * HD + 8 * half;
 #pragma unroll
-        for (int u = 0; u < UT; ++u)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                *(f32x4 *)(part + 32 * u + 8 * q + 4 * half) =
-                    f32x4{oacc[u][4 * q], oacc[u][4 * q + 1], oacc[u][4 * q + 2], oacc[u][4 * q + 3]};
-        if (half == 0) {
-            part[HD] = m2;
-            part[HD + 1] = l;
+        for (int s = 0; s < KSTEPS; ++s) {
+            float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            if (rvalid) {
+                const f32x4 t0 = *(const f32x4 *)(qp + 16 * s), t1 = *(const f32x4 *)(qp + 16 * s + 4);
+                v[0] = t0[0] * sl2; v[1] = t0[1] * sl2; v[2] = t0[2] * sl2; v[3] = t0[3] * sl2;
+                v[4] = t1[0] * sl2; v[5] = t1[1] * sl2; v[6] = t1[2] * sl2; v[7] = t1[3] * sl2;
+            }
+            split3x8(v, q3[s]);
         }
     }
+
+    f32x16 oacc[UT];
+#pragma unroll
+    for (int u = 0; u < UT; ++u) oacc[u] = f32x16{};
+    float m2 = -INFINITY, l = 0.f;
+    for (int t0 = start; t0 < end; t0 += 64) {
+        __syncthreads();  // the previous tile's reads are done
+        stage();
+        __syncthreads();
+        if (t0 + 64 < end) fetch(t0 + 64);
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {
+            f32x16 sacc = f32x16{}, slow = f32x16{};
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) {
+                const int r = 32 * tt + n;
+                const uint16_t *kp = ks + r * HD + (((2 * s + half) ^ (r % CPR)) << 3);
+                const bf16x8 k0 = *(const bf16x8 *)kp, k1 = *(const bf16x8 *)(kp + 64 * HD),
+                             k2 = *(const bf16x8 *)(kp + 2 * 64 * HD);
+                slow = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k2, q3[s][0], slow, 0, 0, 0);
+                sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k0, q3[s][0], sacc, 0, 0, 0);
+                slow = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k1, q3[s][1], slow, 0, 0, 0);
+                slow = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k0, q3[s][2], slow, 0, 0, 0);
+                slow = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k1, q3[s][0], slow, 0, 0, 0);
+                slow = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k0, q3[s][1], slow, 0, 0, 0);
+            }
+            sacc += slow;
+            // Masks, online softmax and delayed rescaling: attn_prefill_kernel's.
+            const int h0 = t0 + 32 * tt;
+            if (h0 + 31 > first_pos || h0 + 32 > end) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int p = h0 + krow_of(8 * (r >> 2) + 4 * half + (r & 3));
+                    if (p > my_pos || p >= end) sacc[r] = -INFINITY;
+                }
+            }
+            float tmax = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, sacc[r]);
+            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+            const bool raise = tmax > m2 + 8.0f;
+            if (__any(raise)) {
+                const float mnew = raise ? tmax : m2;
+                const float alpha = __builtin_amdgcn_exp2f(m2 - mnew);  // 1 where not raised, 0 from -inf
+                l *= alpha;
+#pragma unroll
+                for (int u = 0; u < UT; ++u)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) oacc[u][r] *= alpha;
+                m2 = mnew;
+            }
+            const float mref = m2 == -INFINITY ? 0.f : m2;
+            float tsum = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float pv = __builtin_amdgcn_exp2f(sacc[r] - mref);
+                sacc[r] = pv;
+                tsum += pv;
+            }
+            tsum += __shfl_xor(tsum, 32, 64);
+            l += tsum;
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2) {
+                float pv[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) pv[j] = sacc[8 * s2 + j];
+                bf16x8 p3[3];
+                split3x8(pv, p3);
+#pragma unroll
+                for (int u = 0; u < UT; ++u) {
+                    const int d = 32 * u + n;
+                    const uint16_t *vp = vt + d * LDV + vcol(d, 32 * tt + 16 * s2 + 8 * half);
+                    const bf16x8 v0 = *(const bf16x8 *)vp, v1 = *(const bf16x8 *)(vp + HD * LDV),
+                                 v2 = *(const bf16x8 *)(vp + 2 * HD * LDV);
+                    oacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v2, p3[0], oacc[u], 0, 0, 0);
+                    oacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, p3[1], oacc[u], 0, 0, 0);
+                    oacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v0, p3[2], oacc[u], 0, 0, 0);
+                    oacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v1, p3[0], oacc[u], 0, 0, 0);
+                    oacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v0, p3[1], oacc[u], 0, 0, 0);
+                    oacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v0, p3[0], oacc[u], 0, 0, 0);
+                }
+            }
+        }
+    }
+    if (!rvalid) return;
+    store_prefill_rows<HD>(a, oacc, m2, l, part, (size_t)row * a.q_heads * HD + (size_t)head * HD, S, half);
 }
 
 // Merges the splits of one (row, q head) of attn_prefill_kernel in split
@@ -987,8 +1234,20 @@ template <int HD, int G>
 int launch_prefill_hg(const AttnJob &j, const AttnArgs &a, int S, hipStream_t s) {
     constexpr int RW = 32 / G;
     const int rb = (int)((j.rows + 4 * RW - 1) / (4 * RW));
-    hipLaunchKernelGGL((attn_prefill_kernel<HD, G>), dim3(rb, j.g.kv_heads, S), dim3(kThreads), 0, s, a, (int)j.rows,
-                       S, j.span);
+    if (j.g.kv_f32) {
+        constexpr size_t lds = prefill_f32_lds_bytes<HD>();
+        static bool attr_set = false;
+        if (!attr_set) {
+            CHIP_CHECK(hipFuncSetAttribute((const void *)attn_prefill_f32_kernel<HD, G>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            attr_set = true;
+        }
+        hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, G>), dim3(rb, j.g.kv_heads, S), dim3(kThreads), lds, s, a,
+                           (int)j.rows, S, j.span);
+    } else {
+        hipLaunchKernelGGL((attn_prefill_kernel<HD, G>), dim3(rb, j.g.kv_heads, S), dim3(kThreads), 0, s, a,
+                           (int)j.rows, S, j.span);
+    }
     CHIP_CHECK(hipGetLastError());
     if (S > 1) {
         const int items = (int)j.rows * j.q_heads;
@@ -1097,9 +1356,10 @@ int attention_prefill_splits(size_t ctx, int span) {
 // prefill) 19,130 / 14,155 tok/s with 1,024, 20,418 / 15,737 with 4,096;
 // on 512-row chunks at up to 8K keys (Llama-3-8B) 20,766 tok/s with 1,024,
 // 19,178 with 4,096. Capacity / 8 picks 4,096 for the 33K cache and 1,024
-// for the 8K one.
-int attention_prefill_span(size_t kv_capacity) {
-    int span = kDefaultPrefillSpan;
+// for the 8K one. The f32 kernel runs one block per CU and a tile takes it
+// about three times as long, so short caches take spans from 256 on.
+int attention_prefill_span(size_t kv_capacity, bool kv_f32) {
+    int span = kv_f32 ? kF32PrefillSpan : kDefaultPrefillSpan;
     while ((size_t)span * 2 <= kv_capacity / 8 && span < (1 << 20)) span *= 2;
     return span;
 }
@@ -1110,7 +1370,7 @@ bool attention_decode_fuses_rope(const KvGeom &g, int q_heads, int rotary_dim) {
 }
 
 bool attention_prefill_on_mfma(const KvGeom &g, int q_heads) {
-    return !g.kv_f32 && (g.head_dim == 64 || g.head_dim == 128) && g.kv_heads > 0 && q_heads % g.kv_heads == 0 &&
+    return (g.head_dim == 64 || g.head_dim == 128) && g.kv_heads > 0 && q_heads % g.kv_heads == 0 &&
            q_heads / g.kv_heads <= 8;
 }
 

@@ -152,6 +152,8 @@ int launch_gather_rows(const uint8_t *src, uint8_t *dst, const int32_t *map, siz
 // Keys per split of the matrix-core chunked prefill when the caller names
 // no span (attention_prefill_span gives a model's).
 constexpr int kDefaultPrefillSpan = 1024;
+// Shortest span over an f32 cache.
+constexpr int kF32PrefillSpan = 256;
 
 struct AttnJob {
     const float *q = nullptr;
@@ -165,7 +167,7 @@ struct AttnJob {
     const int32_t *pos_dev = nullptr;
     int splits = 1;
     float *part = nullptr;  // partial buffer (splits > 1)
-    // Chunked prefill (host offset): BF16 KV with head_dim 64/128 runs on the
+    // Chunked prefill (host offset): head_dim 64/128 runs on the
     // matrix cores with attention_prefill_splits(offset + rows) splits and
     // ignores `splits`; part must then hold part_floats >= the partials.
     bool prefill = false;
@@ -197,8 +199,9 @@ int attention_decode_splits(size_t ctx, int kv_heads, size_t rows, bool kv_f32);
 int attention_max_splits();
 int attention_prefill_splits(size_t ctx, int span = kDefaultPrefillSpan);
 // A model's prefill span from its KV capacity: the largest power of two at
-// most capacity / 8, and at least kDefaultPrefillSpan.
-int attention_prefill_span(size_t kv_capacity);
+// most capacity / 8, and at least kDefaultPrefillSpan (f32 cache:
+// kF32PrefillSpan).
+int attention_prefill_span(size_t kv_capacity, bool kv_f32);
 bool attention_prefill_on_mfma(const KvGeom &g, int q_heads);
 
 // Greedy argmax (ties -> last index, total order) of logits[n]; writes the

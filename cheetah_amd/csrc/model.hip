@@ -42,7 +42,6 @@ using namespace chip;
 namespace {
 
 constexpr int kPageSize = 64;
-constexpr int kPrefillSplits = 16;
 
 struct DevAlloc {
     std::vector<void *> ptrs;
@@ -670,11 +669,10 @@ int init_instance(cheetah_hip_model *m) {
     CHIP_TRY(m->mem.alloc(&m->qrot, R * qd));
     CHIP_TRY(m->mem.alloc(&m->act, R * c.intermediate_size));
     CHIP_TRY(m->mem.alloc(&m->logits, c.vocab_size));
-    // Prefill partials: the fixed VALU split count, or the matrix-core
-    // kernel's span splits at full capacity; decode: attention_max_splits.
-    const size_t prefill_splits =
-        std::max((size_t)kPrefillSplits,
-                 (size_t)attention_prefill_splits(sh.kv_capacity, attention_prefill_span(sh.kv_capacity)));
+    // Prefill partials: the span splits at full capacity; decode:
+    // attention_max_splits.
+    const size_t prefill_splits = (size_t)attention_prefill_splits(
+        sh.kv_capacity, attention_prefill_span(sh.kv_capacity, sh.kv_f32 != 0));
     const size_t part_rows = std::max(R * prefill_splits, (size_t)attention_max_splits());
     m->part_floats = part_rows * c.q_heads * (c.head_dim + 2);
     CHIP_TRY(m->mem.alloc(&m->part, m->part_floats));
@@ -992,11 +990,6 @@ int enqueue_chunk(cheetah_hip_model *m, const uint32_t *tokens_dev, size_t rows,
     hipStream_t s = m->stream;
     const size_t H = c.hidden_size;
     CHIP_TRY(launch_embed(sh.embed, H, tokens_dev, rows, m->hidden, s));
-    // A fixed split count makes each row's split boundaries a function of its
-    // own context length only, so a position's attention output does not
-    // depend on how the prompt was cut into chunks (KV continuation stays
-    // bit-exact, decoder.rs:1710-1728).
-    const size_t splits = kPrefillSplits;
     // A residual GEMM that split K leaves its chunk sums in gemm_ws; the
     // reduction then runs fused with the RMSNorm that reads its output.
     int down_chunks = 0;
@@ -1039,17 +1032,16 @@ int enqueue_chunk(cheetah_hip_model *m, const uint32_t *tokens_dev, size_t rows,
         aj.q_heads = (int)c.q_heads;
         aj.rows = rows;
         aj.offset = pos;
-        aj.splits = (int)splits;
         aj.part = m->part;
         aj.part_floats = m->part_floats;
         aj.prefill = true;
-        aj.span = attention_prefill_span(m->sh->kv_capacity);
-        // The matrix-core prefill writes the o_proj input halves itself.
-        const bool halves = attention_prefill_on_mfma(aj.g, aj.q_heads);
-        if (halves) {
-            aj.out_hi = m->xh;
-            aj.out_lo = m->xl;
-        }
+        // Absolute spans of positions, fixed per model: a position's attention
+        // output does not depend on how the prompt was cut into chunks (KV
+        // continuation stays bit-exact, decoder.rs:1710-1728).
+        aj.span = attention_prefill_span(sh.kv_capacity, sh.kv_f32 != 0);
+        // The prefill attention writes the o_proj input halves itself.
+        aj.out_hi = m->xh;
+        aj.out_lo = m->xl;
         CHIP_TRY(launch_attention(aj, s));
         GemmJob o;
         o.w = L.o;
@@ -1060,7 +1052,6 @@ int enqueue_chunk(cheetah_hip_model *m, const uint32_t *tokens_dev, size_t rows,
         o.epi = EPI_RESIDUAL;
         o.ws = m->gemm_ws;
         o.ws_floats = m->gemm_ws_floats;
-        if (!halves) CHIP_TRY(launch_split_bf16(m->attn, rows * (size_t)(sh.q_dim()), m->xh, m->xl, s));
         o.xh = m->xh;
         o.xl = m->xl;
         int o_chunks = 0;

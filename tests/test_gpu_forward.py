@@ -95,6 +95,24 @@ def test_tiny_greedy_32_steps_token_exact(hip, oracle, shape, kv):
     assert [first] + rest.tolist() == ref_tokens
 
 
+@pytest.mark.parametrize("shape", TINY, ids=lambda s: s.name)
+def test_f32_kv_prefill_attention_tile_and_span_edges(hip, oracle, shape):
+    """f32-cache prefill attention at the edges of its 64-key tiles, 256-key
+    spans (capacity below 4,096) and row blocks, with a ragged chunk split.
+    The attention itself is exact to f32 rounding; what is left against the
+    oracle is the GEMMs' hi/lo input split: 2^-17 per product, averaged over a
+    dot product, through 2 layers of 4 GEMMs on the largest logit: 5e-5."""
+    g = hip.HipForward(shape, weights(shape), kv="f32", kv_capacity=640, max_chunk_rows=160)
+    r = oracle.RefModel(shape, weights(shape))
+    toks = synth.make_tokens(shape.vocab_size, 521, seed=21)
+    for n, chunk in ((2, 160), (63, 160), (65, 64), (255, 33), (257, 160), (521, 147)):
+        g.clear_cache()
+        r.clear_cache()
+        got = g.forward(toks[:n], 0, chunk_rows=chunk)
+        ref = r.forward(toks[:n], 0, chunk_rows=256)
+        assert rel_err(got, ref) < 5e-5, (n, chunk)
+
+
 @pytest.mark.parametrize("kv", ["bf16", "f32"])
 def test_kv_continuation_bit_exact_on_device(hip, kv):
     # decoder.rs:1710-1728: prefill in one call == prefill in two calls.
