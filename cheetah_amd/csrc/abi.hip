@@ -178,7 +178,7 @@ int cheetah_hip_gemv_q4(const uint8_t *w, size_t rows, size_t cols, const float 
 static int gemm_scratch(size_t rows, size_t cols, size_t n, GemmJob &j) {
     static thread_local float *ws = nullptr;
     static thread_local size_t ws_floats = 0;
-    const size_t need = gemm_split_workspace_floats(rows, cols, n, false);
+    const size_t need = gemm_workspace_floats(j.w.fmt, rows, cols, n, false);
     if (need > ws_floats) {
         CHIP_CHECK(hipStreamSynchronize(g_stream));
         if (ws) CHIP_CHECK(hipFree(ws));
@@ -386,6 +386,7 @@ int cheetah_hip_time_gemm(uint32_t fmt, const void *const *w, size_t nbuf, size_
     for (size_t i = 0; i < nbuf; ++i)
         if (!w[i]) return fail("HIP backend: time_gemm with a null weight buffer.");
     GemmJob j;
+    j.w = WMat{(int)fmt, (const uint8_t *)w[0], rows, cols};
     j.x = x;
     j.n = n;
     j.y = y;

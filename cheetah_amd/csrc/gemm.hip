@@ -9,10 +9,9 @@
 // so two v_mfma_f32_32x32x16_bf16 per k-step carry x to ~2^-17 relative
 // error (f32 accumulation), instead of bf16's 2^-9.
 //
-// Tiling: a block of 4 or 8 waves (2 x 2 or 4 x 2) computes 64 or 128
-// tokens x 128 weight rows, each wave 32 tokens x 64 rows (the register-
-// staged fallback also 64 x 64 per wave); K advances 32 per LDS stage, the
-// next stages' copies in flight during the MFMAs.
+// Tiling: blocks of 64 x 128, 128 x 128 or 128 x 256 (tokens x weight rows),
+// chosen with the K split by ring_plan; K advances 32 per LDS stage, the next
+// stages' copies in flight during the MFMAs.
 //
 // Accumulation order: K is cut into chunks of a depth fixed by K alone; each
 // chunk is accumulated from zero. A single matrix's n chunk sums are folded
@@ -260,12 +259,12 @@ __device__ __forceinline__ void epilogue(const GArgs &a, int m, int n, float v, 
 // rows m = mbase + 32 i + 8 (q / 4) + 4 (lane / 32) + q % 4. The column's scale
 // and bias, then a 32-row block's residuals, are loaded before any store (one
 // wait instead of one per output); each output's arithmetic is epilogue's.
-template <bool DUAL, int MT>
-__device__ __forceinline__ void epilogue_tile(const GArgs &a, const f32x16 (&tot)[MT][2],
-                                              const f32x16 (&tot2)[DUAL ? MT : 1][2], int mbase, int nbase, int lane) {
+template <bool DUAL, int MT, int NJ = 2>
+__device__ __forceinline__ void epilogue_tile(const GArgs &a, const f32x16 (&tot)[MT][NJ],
+                                              const f32x16 (&tot2)[DUAL ? MT : 1][NJ], int mbase, int nbase, int lane) {
     const bool resid = !DUAL && a.epi == EPI_RESIDUAL;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < NJ; ++j) {
         const int n = nbase + 32 * j + (lane & 31);
         if (n >= a.N) continue;
         const float scn = a.sc ? a.sc[n] : 1.0f;
@@ -312,11 +311,11 @@ __device__ __forceinline__ void epilogue_tile(const GArgs &a, const f32x16 (&tot
 // round-robin) run on one XCD: each weight tile streams from HBM about once
 // and the block's neighbours find it in that XCD's L2, instead of every token
 // tile re-reading the whole matrix.
-__device__ __forceinline__ void tile_of(int nN, int nM, int &n0, int &m0, int BMt) {
+__device__ __forceinline__ void tile_of(int nN, int nM, int &n0, int &m0, int BMt, int BNt = BN) {
     const int total = nN * nM, bid = blockIdx.x;
     const int lid = total % 8 == 0 ? (bid % 8) * (total / 8) + bid / 8 : bid;
     m0 = (lid % nM) * BMt;
-    n0 = (lid / nM) * BN;
+    n0 = (lid / nM) * BNt;
 }
 
 // blockIdx: x = output tile (tile_of), z = chunk (split-K) or 0.
@@ -467,39 +466,9 @@ __global__ __launch_bounds__(kThreads) void gemm_reduce_kernel(GArgs a);
 // s_waitcnt immediate waiting until at most n vector-memory ops are pending.
 constexpr int vm_wait_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
 
-// ---------------------------------------------------------------------------
-// Ring GEMM, every weight format (x pre-split, K % 32 == 0). Per 32-wide K
-// stage the block's x halves and its raw weight bytes (BF16 rows, Q8 codes,
-// Q4 nibbles) go global -> LDS by buffer loads that write LDS directly: a
-// lane's source offset is fixed for the whole launch and the stage's K
-// offset is a scalar, so issuing a stage costs no vector instructions. The
-// ring holds NS = 4 stages (6 measured no faster); stage s + NS - 2 is issued
-// while stage s computes.
-// Q8/Q4 codes of stage s + 1 are converted to BF16 (exactly) once per block,
-// 16 (4 waves) or 8 (8 waves) per thread, into one of three converted tiles
-// after stage s's MFMAs;
-// BF16 weights are read straight from the ring. One barrier per stage. The
-// MFMA sequence per output and the chunk folds are those of gemm_kernel, so
-// the results are the same bits.
-// ---------------------------------------------------------------------------
+// Raw weight bytes per row and 32-column stage.
 template <int FMT>
-constexpr int ring_w_row_bytes() { return FMT == FMT_BF16 ? 64 : FMT == FMT_Q8 ? 32 : 16; }
-
-// Tokens per block: WV waves as WV / 2 x 2, each 32 MT tokens x 64 rows.
-template <int MT, int WV>
-constexpr int ring_bm() { return 32 * MT * (WV / 2); }
-
-template <int FMT, bool DUAL, int MT, int NS, int WV>
-constexpr size_t ring_lds_bytes() {
-    constexpr size_t slot = 2 * ring_bm<MT, WV>() * 64 + (DUAL ? 2 : 1) * BN * ring_w_row_bytes<FMT>();
-    return NS * slot + (FMT == FMT_BF16 ? 0 : 3 * (DUAL ? 2 : 1) * BN * 64);
-}
-
-// Weight copy granule (bytes per lane) of the ring: Q4 rows are only 4-byte
-// aligned; Q8 stages are copied 4 bytes a lane where 16 would leave some of
-// 8 waves without a copy (every wave must issue the same count).
-template <int FMT, int WV>
-constexpr int ring_w_granule() { return FMT == FMT_Q4 ? 4 : (FMT == FMT_Q8 && WV == 8) ? 4 : 16; }
+constexpr int w_row_bytes() { return FMT == FMT_BF16 ? 64 : FMT == FMT_Q8 ? 32 : 16; }
 
 typedef __attribute__((address_space(3))) void lds_void;
 
@@ -511,34 +480,81 @@ __device__ __forceinline__ void buf_to_lds(__amdgpu_buffer_rsrc_t r, void *lds, 
     else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 4, voffset, soffset, 0, 0);
 }
 
-template <int FMT, bool DUAL, int MT, int NS, int WV>
-__global__ __launch_bounds__(64 * WV) void gemm_ring_kernel(GArgs a, int split) {
-    constexpr int NT = 64 * WV;                      // threads
-    constexpr int BM = ring_bm<MT, WV>();
-    constexpr int XB = BM * 64;                      // bytes of one x half tile (BM rows x 32 BF16)
-    constexpr int WRB = ring_w_row_bytes<FMT>();     // raw weight bytes per row and stage
-    constexpr int WB = BN * WRB;                     // raw weight bytes per matrix and stage
-    constexpr int NWM = DUAL ? 2 : 1;
-    constexpr int SLOT = 2 * XB + NWM * WB;
+// ---------------------------------------------------------------------------
+// Ring GEMM, every weight format (x pre-split, K % 32 == 0): WM x WN waves of
+// 32 MT tokens x 64 weight rows (DUAL: 32 gate and the matching 32 up rows).
+// Per 32-wide K stage the block's x halves and its raw weight bytes (BF16
+// rows, Q8 codes, Q4 nibbles) go global -> LDS by buffer loads that write LDS
+// directly: a lane's source offset is fixed for the whole launch and the
+// stage's K offset is a scalar, so a copy costs no vector instructions. The
+// ring holds NS stages. Q8/Q4 codes are converted to BF16 (exactly) once per
+// block, two stages ahead, into one of two converted tiles; BF16 weights are
+// read straight from the ring. One barrier per stage.
+//
+// Fragments run one k-step (16 columns) ahead: the LDS reads of k-step s + 1
+// and the copies of a later stage sit between the MFMAs of k-step s, so
+// neither a read's latency nor a burst of copies holds the matrix cores, and
+// the barrier falls inside a stage's MFMAs. Iteration st (fragments F0 read):
+//   MFMAs of F0, reading F1(st); wait for this wave's copies of the next
+//   stage(s); barrier; MFMAs of F1, reading F0(st + 1) and issuing stage
+//   st + NS - 1 (its slot held stage st - 1, whose reads every wave finished
+//   before the barrier); Q8/Q4: convert stage st + 2 (its tile held stage st).
+// The MFMA sequence per output and the chunk folds are those of gemm_kernel,
+// so the results are the same bits whatever the tile.
+//
+// Bound: the matrix cores, at the clock they leave (51 % busy over a wave's
+// life at 2,048 tokens x 4096 x 4096; a large BF16 product of the BLAS library
+// reaches 1.2 PFLOP/s on this card, this kernel 1.02 executed). Tiles, per
+// block: 128 tokens x 256 rows on 8 waves of 64 x 64 (an LDS byte feeds 1.5
+// times the MFMAs of 32 x 64, and the block's L2 traffic per MFMA is 2/3 of
+// 128 x 128); 128 x 128 on 8 waves of 32 x 64; 64 x 128 on 4 waves, two blocks
+// per CU. Before, 8-wave 128 x 128 blocks read a whole stage's fragments after
+// its barrier. TFLOP/s (x split included), before -> now: 14336 x 4096 at 512
+// tokens BF16 359 -> 504, Q8 315 -> 457, Q4 310 -> 450; 4096 x 4096 at 2,048
+// tokens 366 -> 509 / 338 -> 467 / 347 -> 475; 3584 x 18944 at 1,024 407 ->
+// 509 / 366 -> 441 / 354 -> 438. Measured and not kept: 128 x 128 on 4 waves
+// of 64 x 64, two blocks per CU (393 TFLOP/s at 2,048 tokens); rings one or
+// two stages deeper (even); the first half's total in memory instead of
+// registers (471 against 509); the copies in one burst after the barrier (423).
+// ---------------------------------------------------------------------------
+template <int FMT, int MT, int WM, int WN, int NS>
+constexpr size_t ring_lds_bytes() {
+    constexpr size_t bn = 64 * WN, slot = 2 * (32 * MT * WM) * 64 + bn * w_row_bytes<FMT>();
+    return NS * slot + (FMT == FMT_BF16 ? 0 : 2 * bn * 64);
+}
+
+template <int FMT, bool DUAL, int MT, int WM, int WN, int NS, int QG>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_ring_kernel(GArgs a, int split) {
+    constexpr int WV = WM * WN, NT = 64 * WV;
+    constexpr int BM = 32 * MT * WM, BNR = 64 * WN;  // tokens, weight rows of the block (DUAL: half of each matrix)
+    constexpr int BNO = DUAL ? BNR / 2 : BNR;        // output columns of the block
+    constexpr int XB = BM * 64;
+    constexpr int WRB = w_row_bytes<FMT>();
+    constexpr int WB = BNR * WRB;
+    constexpr int SLOT = 2 * XB + WB;
     constexpr bool CONV = FMT != FMT_BF16;
-    constexpr int WCB = BN * 64;                     // one converted BF16 weight tile
-    constexpr int GW = ring_w_granule<FMT, WV>();    // weight copy granule
-    constexpr int NIX = XB / 1024;                   // 1 KB copies per x half
-    constexpr int NIW = WB / (64 * GW);              // copies per weight matrix
-    constexpr int D = 2 * NIX / WV + NWM * NIW / WV; // copies per wave and stage
-    constexpr int CPT = BN * 32 / NT;                // codes each thread converts per matrix and stage
+    constexpr int WCB = BNR * 64;
+    // Weight copy granule (bytes per lane): Q4 rows are only 4-byte aligned, Q8
+    // ones where the row count is odd (QG = 4); Q8 also 4 where 16 would leave
+    // some waves without a copy.
+    constexpr int GW = FMT == FMT_Q4 || (FMT == FMT_Q8 && (QG == 4 || WB / 1024 % WV)) ? 4 : 16;
+    constexpr int NIX = XB / 1024, NIW = WB / (64 * GW);
+    constexpr int D = 2 * NIX / WV + NIW / WV;       // copies per wave and stage
+    constexpr int CPT = BNR * 32 / NT;               // codes each thread converts per stage
     static_assert(NIX % WV == 0 && NIW % WV == 0, "copies must split evenly over the waves");
     static_assert(CPT == 8 || CPT == 16, "8 or 16 codes per converting thread");
-    static_assert(NS >= 4, "the converted weights trail the ring by one stage");
+    static_assert(NS >= (CONV ? 4 : 3), "stages in flight behind the one computed");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     uint8_t *ring = smem;
-    uint8_t *wcv = smem + NS * SLOT;  // CONV: [3][NWM] converted tiles
+    uint8_t *wcv = smem + NS * SLOT;  // CONV: [2] converted tiles
 
     int n0, m0;
-    tile_of((a.N + BN - 1) / BN, (a.M + BM - 1) / BM, n0, m0, BM);
+    tile_of((a.N + BNO - 1) / BNO, (a.M + BM - 1) / BM, n0, m0, BM, BNO);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int wm = (wave >> 1) * 32 * MT, wn = (wave & 1) * 64;
+    const int wm = (wave / WN) * 32 * MT, wj = wave % WN;
+    // Weight-tile row of the wave's column group j.
+    auto wrow = [&](int j) { return DUAL ? j * (BNR / 2) + 32 * wj : 64 * wj + 32 * j; };
     // split 0: all of K; 1: chunk blockIdx.z; 2: half blockIdx.z of a single
     // matrix's chunks (the first hc chunks, then the rest).
     const int hc = (a.nchunks + 1) / 2;
@@ -553,9 +569,6 @@ __global__ __launch_bounds__(64 * WV) void gemm_ring_kernel(GArgs a, int split) 
     const __amdgpu_buffer_rsrc_t rw2 =
         __builtin_amdgcn_make_buffer_rsrc((void *)(DUAL ? a.w2 : a.w), (short)0, wbytes, 0x00020000);
 
-    // Per-lane source offsets of this wave's copies (fixed for the launch):
-    // x copy q covers rows 16q..16q+15, lane -> row 16q + lane/4 and 16-byte
-    // chunk swz(row, lane % 4) of the stage's 32 columns.
     int xoff[NIX / WV], woff[NIW / WV];
 #pragma unroll
     for (int i = 0; i < NIX / WV; ++i) {
@@ -563,6 +576,10 @@ __global__ __launch_bounds__(64 * WV) void gemm_ring_kernel(GArgs a, int split) 
         const int m = min(m0 + r, a.M - 1);  // rows past M feed only unstored outputs
         xoff[i] = (m * a.K + 8 * swz(r, lane & 3)) * 2;
     }
+    // Weight copy q covers rows RPC q .. RPC q + RPC - 1 of the tile; with
+    // DUAL the first half of the copies reads the gate matrix, the rest up.
+    constexpr int RPC = 64 * GW / WRB;
+    auto w_up = [&](int i) { return DUAL && (wave + WV * i) * RPC >= BNR / 2; };
 #pragma unroll
     for (int i = 0; i < NIW / WV; ++i) {
         const int q = wave + WV * i;
@@ -571,238 +588,231 @@ __global__ __launch_bounds__(64 * WV) void gemm_ring_kernel(GArgs a, int split) 
         else if constexpr (FMT == FMT_Q8 && GW == 16) { r = 32 * q + (lane >> 1); byte = 16 * (lane & 1); }
         else if constexpr (FMT == FMT_Q8) { r = 8 * q + (lane >> 3); byte = 4 * (lane & 7); }
         else { r = 16 * q + (lane >> 2); byte = 4 * (lane & 3); }
-        const int n = min(n0 + r, a.N - 1);
+        const int n = min(n0 + (w_up(i) ? r - BNR / 2 : r), a.N - 1);
         woff[i] = n * (int)a.stride + byte;
     }
-    // Stage st's copies into ring slot st % NS (stages past the range re-read
-    // the last one into a free slot, so every wave issues the same count).
-    auto issue = [&](int st) {
+    // Copy d (0 .. D - 1) of this wave's copies of stage st into ring slot
+    // st % NS (stages past the range re-read the last one into a free slot,
+    // so every wave issues the same count).
+    auto issue1 = [&](int st, int d) {
         const int k0 = kbeg + min(st, nst - 1) * BK;
         uint8_t *slot = ring + (st % NS) * SLOT;
-        const int kx = k0 * 2;
-        const int kw = FMT == FMT_BF16 ? k0 * 2 : FMT == FMT_Q8 ? k0 : k0 / 2;
-#pragma unroll
-        for (int i = 0; i < NIX / WV; ++i) {
-            const int q = wave + WV * i;
-            buf_to_lds<16>(rxh, slot + 1024 * q, xoff[i], kx);
-            buf_to_lds<16>(rxl, slot + XB + 1024 * q, xoff[i], kx);
-        }
-#pragma unroll
-        for (int i = 0; i < NIW / WV; ++i) {
-            const int q = wave + WV * i;
-            buf_to_lds<GW>(rw, slot + 2 * XB + 64 * GW * q, woff[i], kw);
-            if constexpr (DUAL)
-                buf_to_lds<GW>(rw2, slot + 2 * XB + WB + 64 * GW * q, woff[i], kw);
+        constexpr int XI = NIX / WV;
+        if (d < 2 * XI) {
+            const int i = d >> 1, q = wave + WV * i;
+            if (d & 1) buf_to_lds<16>(rxl, slot + XB + 1024 * q, xoff[i], k0 * 2);
+            else buf_to_lds<16>(rxh, slot + 1024 * q, xoff[i], k0 * 2);
+        } else {
+            const int i = d - 2 * XI;
+            const int kw = FMT == FMT_BF16 ? k0 * 2 : FMT == FMT_Q8 ? k0 : k0 / 2;
+            uint8_t *dst = slot + 2 * XB + 64 * GW * (wave + WV * i);
+            if (w_up(i)) buf_to_lds<GW>(rw2, dst, woff[i], kw);
+            else buf_to_lds<GW>(rw, dst, woff[i], kw);
         }
     };
-    // Q8/Q4: stage st's codes -> BF16 tile(s) wcv[st % 3], thread t: row
-    // t / (32 / CPT), codes CPT (t % (32 / CPT)) .. + CPT - 1, written in the
-    // swizzled layout the MFMA reads.
-    // The raw codes are read by inline assembly: the compiler, which cannot
-    // tell these reads from the ring's in-flight copies, would otherwise wait
-    // for every copy (all NS stages) before them. The copies they need were
-    // awaited explicitly.
+    // Stage st's codes -> BF16 tile wcv[st % 2], thread t: row t / TPR, codes
+    // CPT (t % TPR) .. + CPT - 1, written in the swizzled layout the MFMA
+    // reads. The raw codes are read by inline assembly: the compiler, which
+    // cannot tell these reads from the ring's in-flight copies, would
+    // otherwise wait for every copy before them. The copies they need were
+    // awaited explicitly, and each read waits for its data inside its own asm
+    // statement, so no use of the result can be scheduled ahead of the wait.
     auto convert = [&](int st) {
-        constexpr int TPR = 32 / CPT;  // threads per row
-        constexpr int RB = FMT == FMT_Q8 ? CPT : CPT / 2;  // raw bytes per thread
+        constexpr int TPR = 32 / CPT, RB = FMT == FMT_Q8 ? CPT : CPT / 2;
         const uint8_t *slot = ring + (st % NS) * SLOT + 2 * XB;
         const int row = threadIdx.x / TPR, h = threadIdx.x % TPR;
-        // (Each read waits for its data inside its own asm statement, so no
-        // use of the result can be scheduled ahead of the wait.)
-        u32x4 rv[NWM];
-#pragma unroll
-        for (int mi = 0; mi < NWM; ++mi) {
-            const uint32_t addr = (uint32_t)(uintptr_t)(slot + mi * WB + row * WRB + RB * h);
-            if constexpr (RB == 16) {
-                asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(rv[mi]) : "v"(addr) : "memory");
-            } else if constexpr (RB == 8) {
-                uint2 t;
-                asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(t) : "v"(addr) : "memory");
-                rv[mi] = u32x4{t.x, t.y, 0u, 0u};
-            } else {
-                uint32_t t;
-                asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(t) : "v"(addr) : "memory");
-                rv[mi] = u32x4{t, 0u, 0u, 0u};
-            }
+        const uint32_t addr = (uint32_t)(uintptr_t)(slot + row * WRB + RB * h);
+        u32x4 rv;
+        if constexpr (RB == 16) {
+            asm volatile("ds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(rv) : "v"(addr) : "memory");
+        } else if constexpr (RB == 8) {
+            uint2 t;
+            asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(t) : "v"(addr) : "memory");
+            rv = u32x4{t.x, t.y, 0u, 0u};
+        } else {
+            uint32_t t;
+            asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(t) : "v"(addr) : "memory");
+            rv = u32x4{t, 0u, 0u, 0u};
         }
+        float f[CPT];
+        if constexpr (FMT == FMT_Q8) {
 #pragma unroll
-        for (int mi = 0; mi < NWM; ++mi) {
-            float f[CPT];
-            if constexpr (FMT == FMT_Q8) {
-                const u32x4 v = rv[mi];
+            for (int q = 0; q < CPT; ++q) f[q] = (float)(int)(int8_t)(rv[q >> 2] >> (8 * (q & 3)));
+        } else {
 #pragma unroll
-                for (int q = 0; q < CPT; ++q) f[q] = (float)(int)(int8_t)(v[q >> 2] >> (8 * (q & 3)));
-            } else {
+            for (int h2 = 0; h2 < CPT / 8; ++h2) {
                 // 16 x code: each nibble moved to the top of a byte, read as
                 // int8 in one instruction (exact in BF16; the chunk sums are
                 // scaled back by 1/16, exactly).
-#pragma unroll
-                for (int h2 = 0; h2 < CPT / 8; ++h2) {
-                    const uint32_t wd = rv[mi][h2];
-                    const uint32_t ev = (wd << 4) & 0xF0F0F0F0u, od = wd & 0xF0F0F0F0u;
-                    f[8 * h2 + 0] = sbyte_f32<0>(ev);
-                    f[8 * h2 + 1] = sbyte_f32<0>(od);
-                    f[8 * h2 + 2] = sbyte_f32<1>(ev);
-                    f[8 * h2 + 3] = sbyte_f32<1>(od);
-                    f[8 * h2 + 4] = sbyte_f32<2>(ev);
-                    f[8 * h2 + 5] = sbyte_f32<2>(od);
-                    f[8 * h2 + 6] = sbyte_f32<3>(ev);
-                    f[8 * h2 + 7] = sbyte_f32<3>(od);
-                }
-            }
-            uint8_t *dst = wcv + ((st % 3) * NWM + mi) * WCB + row * 64;
-#pragma unroll
-            for (int c = 0; c < CPT / 8; ++c) {
-                bf16x8 b;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) b[e] = (__bf16)f[8 * c + e];
-                *(bf16x8 *)(dst + 16 * swz(row, (CPT / 8) * h + c)) = b;
+                const uint32_t wd = rv[h2];
+                const uint32_t ev = (wd << 4) & 0xF0F0F0F0u, od = wd & 0xF0F0F0F0u;
+                f[8 * h2 + 0] = sbyte_f32<0>(ev);
+                f[8 * h2 + 1] = sbyte_f32<0>(od);
+                f[8 * h2 + 2] = sbyte_f32<1>(ev);
+                f[8 * h2 + 3] = sbyte_f32<1>(od);
+                f[8 * h2 + 4] = sbyte_f32<2>(ev);
+                f[8 * h2 + 5] = sbyte_f32<2>(od);
+                f[8 * h2 + 6] = sbyte_f32<3>(ev);
+                f[8 * h2 + 7] = sbyte_f32<3>(od);
             }
         }
+        uint8_t *dst = wcv + (st & 1) * WCB + row * 64;
+#pragma unroll
+        for (int c = 0; c < CPT / 8; ++c) {
+            bf16x8 b;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) b[e] = (__bf16)f[8 * c + e];
+            *(bf16x8 *)(dst + 16 * swz(row, (CPT / 8) * h + c)) = b;
+        }
     };
-
-    // th: a single matrix's first-half total while the second half runs
-    // (folding in registers over all of K).
-    f32x16 acc[MT][2], acc2[DUAL ? MT : 1][2], tot[MT][2], tot2[DUAL ? MT : 1][2], th[DUAL ? 1 : MT][2];
+    struct Frags {
+        bf16x8 ah[MT], al[MT], bw[2];
+    };
+    // Fragment read d (0 .. NR - 1) of k-step k of stage st.
+    constexpr int NR = 2 + 2 * MT;
+    auto read1 = [&](int st, int k, int d, Frags &f) {
+        const uint8_t *xs = ring + (st % NS) * SLOT;
+        const uint8_t *wt = CONV ? wcv + (st & 1) * WCB : xs + 2 * XB;
+        const int c = 2 * k + (lane >> 5);
+        if (d < 2) {
+            const int r = wrow(d) + (lane & 31);
+            f.bw[d] = *(const bf16x8 *)(wt + r * 64 + 16 * swz(r, c));
+        } else {
+            const int i = (d - 2) % MT, r = wm + 32 * i + (lane & 31);
+            if (d - 2 < MT) f.ah[i] = *(const bf16x8 *)(xs + r * 64 + 16 * swz(r, c));
+            else f.al[i] = *(const bf16x8 *)(xs + XB + r * 64 + 16 * swz(r, c));
+        }
+    };
+    f32x16 acc[MT][2], tot[MT][2];
+    // MFMA t (0 .. 4 MT - 1) of a k-step: the high halves of x, then the low.
+    constexpr int NM = 4 * MT;
+    auto mma1 = [&](const Frags &f, int t) {
+        const int i = (t / 2) % MT, j = t & 1;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t < 2 * MT ? f.ah[i] : f.al[i], f.bw[j], acc[i][j], 0, 0, 0);
+    };
+    // One k-step: the MFMAs of f with the reads of the next k-step into g and
+    // copies d0 .. d1 - 1 of stage sti between them.
+    constexpr int RPM = 2;  // fragment reads per MFMA, until all are issued
+    auto kstep = [&](const Frags &f, Frags &g, int st, int k, int sti, int d0, int d1) {
+#pragma unroll
+        for (int t = 0; t < NM; ++t) {
+            mma1(f, t);
+#pragma unroll
+            for (int d = RPM * t; d < min(RPM * t + RPM, NR); ++d) read1(st, k, d, g);
+#pragma unroll
+            for (int d = d0 + t * (d1 - d0) / NM; d < d0 + (t + 1) * (d1 - d0) / NM; ++d) issue1(sti, d);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            tot[i][j] = f32x16{};
-            if constexpr (DUAL) tot2[i][j] = f32x16{};
-            else th[i][j] = f32x16{};
-        }
+        for (int j = 0; j < 2; ++j) tot[i][j] = f32x16{};
 
+    constexpr int DH = D / 2 + D % 2;  // copies issued in a stage's second k-step
 #pragma unroll
-    for (int st = 0; st < NS - 2; ++st) issue(st);
+    for (int st = 0; st < NS - 1; ++st)
+#pragma unroll
+        for (int d = 0; d < (st == NS - 2 ? DH : D); ++d) issue1(st, d);
+    __builtin_amdgcn_s_waitcnt(vm_wait_imm(D * (CONV ? NS - 4 : NS - 3) + DH));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     if constexpr (CONV) {
-        __builtin_amdgcn_s_waitcnt(vm_wait_imm(D * (NS - 3)));
-        __builtin_amdgcn_s_barrier();
         convert(0);
+        convert(1);
+        __builtin_amdgcn_s_waitcnt(vm_wait_imm(63) & ~(0xF << 8));  // lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
     }
+    Frags f0, f1;
+#pragma unroll
+    for (int d = 0; d < NR; ++d) read1(0, 0, d, f0);
     const int cs = a.chunk / BK;  // stages per accumulation chunk
+    // Stages [s0, s1), whole chunks, folded into tot.
+    auto run = [&](int s0, int s1) {
+        for (int c0 = s0; c0 < s1; c0 += cs) {
+            const int c1 = min(c0 + cs, s1);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
+            for (int st = c0; st < c1; ++st) {
+                kstep(f0, f1, st, 1, st + NS - 2, DH, D);
+                __builtin_amdgcn_s_waitcnt(vm_wait_imm(D * (CONV ? NS - 4 : NS - 3)));
+                __builtin_amdgcn_s_waitcnt(vm_wait_imm(63) & ~(0xF << 8));  // lgkmcnt(0)
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                kstep(f1, f0, st + 1, 0, st + NS - 1, 0, DH);  // past the last stage: stale bytes, unused
+                if constexpr (CONV) convert(st + 2);
+            }
+            constexpr float cs16 = FMT == FMT_Q4 ? 0.0625f : 1.0f;
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) tot[i][j] += FMT == FMT_Q4 ? acc[i][j] * cs16 : acc[i][j];
+        }
+    };
     const bool halves = !DUAL && !split && hc < a.nchunks;
-    for (int c0 = 0; c0 < nst; c0 += cs) {
-        const int c1 = min(c0 + cs, nst);
-        // The second half begins: th = t, t = 0.
-        const bool half_start = halves && c0 == hc * cs;
+    run(0, halves ? hc * cs : nst);
+    f32x16 th[DUAL ? 1 : MT][2];
+    if constexpr (!DUAL) {
+        if (halves) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+            for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                acc[i][j] = f32x16{};
-                if constexpr (DUAL) {
-                    acc2[i][j] = f32x16{};
-                } else if (half_start) {
+                for (int j = 0; j < 2; ++j) {
                     th[i][j] = tot[i][j];
                     tot[i][j] = f32x16{};
                 }
-            }
-        for (int st = c0; st < c1; ++st) {
-            issue(st + NS - 2);
-            // This wave's copies of stage st (and, converting, st + 1) have
-            // landed once only the later stages' copies are pending; after
-            // the barrier every wave's have, and the tile converted in the
-            // previous iteration is visible.
-            __builtin_amdgcn_s_waitcnt(vm_wait_imm(D * (CONV ? NS - 3 : NS - 2)));
-            __builtin_amdgcn_s_waitcnt(vm_wait_imm(63) & ~(0xF << 8));  // lgkmcnt(0)
-            __builtin_amdgcn_s_barrier();
-            const uint8_t *xs = ring + (st % NS) * SLOT;
-            const uint8_t *wt = CONV ? wcv + (st % 3) * NWM * WCB : xs + 2 * XB;
-            const uint8_t *wt2 = wt + (CONV ? WCB : WB);
-            // Every fragment of the stage is read before the first MFMA, so
-            // the LDS latency is paid once per stage, not once per k-step.
-            constexpr int KS = BK / 16;
-            bf16x8 ah[KS][MT], al[KS][MT], bw[KS][2], bw2[KS][DUAL ? 2 : 1];
+            run(hc * cs, nst);
 #pragma unroll
-            for (int k = 0; k < KS; ++k) {
-                const int c = 2 * k + (lane >> 5);
+            for (int i = 0; i < MT; ++i)
 #pragma unroll
-                for (int i = 0; i < MT; ++i) {
-                    const int r = wm + 32 * i + (lane & 31);
-                    ah[k][i] = *(const bf16x8 *)(xs + r * 64 + 16 * swz(r, c));
-                    al[k][i] = *(const bf16x8 *)(xs + XB + r * 64 + 16 * swz(r, c));
-                }
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const int r = wn + 32 * j + (lane & 31);
-                    bw[k][j] = *(const bf16x8 *)(wt + r * 64 + 16 * swz(r, c));
-                    if constexpr (DUAL) bw2[k][j] = *(const bf16x8 *)(wt2 + r * 64 + 16 * swz(r, c));
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the MFMAs
-#pragma unroll
-            for (int k = 0; k < KS; ++k)
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[k][i], bw[k][j], acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[k][i], bw[k][j], acc[i][j], 0, 0, 0);
-                        if constexpr (DUAL) {
-                            acc2[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[k][i], bw2[k][j], acc2[i][j], 0, 0, 0);
-                            acc2[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[k][i], bw2[k][j], acc2[i][j], 0, 0, 0);
-                        }
-                    }
-            // Stage st + 1's codes, converted while this stage's MFMAs drain
-            // (measured 2-7 % faster than converting before them).
-            if constexpr (CONV) {
-                if (st + 1 < nst) convert(st + 1);
-            }
+                for (int j = 0; j < 2; ++j) tot[i][j] = th[i][j] + tot[i][j];
         }
-        // Chunk end: t += c (Q4: c = acc / 16, exactly).
-        constexpr float cs16 = FMT == FMT_Q4 ? 0.0625f : 1.0f;
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                tot[i][j] += FMT == FMT_Q4 ? acc[i][j] * cs16 : acc[i][j];
-                if constexpr (DUAL) tot2[i][j] += FMT == FMT_Q4 ? acc2[i][j] * cs16 : acc2[i][j];
-            }
     }
     // Drain the copies of stages past the range before the block exits.
     __builtin_amdgcn_s_waitcnt(vm_wait_imm(0));
     if (!split) {
         if constexpr (!DUAL) {
-            if (halves) {
+            epilogue_tile<false, MT>(a, tot, reinterpret_cast<const f32x16(&)[1][2]>(tot), m0 + wm, n0 + 64 * wj, lane);
+        } else {
+            f32x16 gt[MT][1], up[MT][1];
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) tot[i][j] = th[i][j] + tot[i][j];
+            for (int i = 0; i < MT; ++i) {
+                gt[i][0] = tot[i][0];
+                up[i][0] = tot[i][1];
             }
+            epilogue_tile<true, MT, 1>(a, gt, up, m0 + wm, n0 + 32 * wj, lane);
         }
-        epilogue_tile<DUAL, MT>(a, tot, tot2, m0 + wm, n0 + wn, lane);
         return;
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        const int n = n0 + wn + 32 * j + (lane & 31);
+        const int n = n0 + (DUAL ? 32 * wj : 64 * wj + 32 * j) + (lane & 31);
         if (n >= a.N) continue;
+        float *ws = a.ws + (DUAL && j ? (size_t)a.nstored * a.M * a.N : 0);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
                 const int m = m0 + wm + 32 * i + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-                if (m >= a.M) continue;
-                const size_t o = ((size_t)blockIdx.z * a.M + m) * a.N + n;
-                a.ws[o] = tot[i][j][q];
-                if constexpr (DUAL) a.ws[(size_t)a.nstored * a.M * a.N + o] = tot2[i][j][q];
+                if (m < a.M) ws[((size_t)blockIdx.z * a.M + m) * a.N + n] = tot[i][j][q];
             }
     }
 }
 
-template <int FMT, bool DUAL, int MT, int WV = 4>
+template <int FMT, bool DUAL, int MT, int WM, int WN, int NS, int QG>
 int launch_ring(const GArgs &a, int split, hipStream_t s) {
-    constexpr int NS = 4, BM = ring_bm<MT, WV>();
-    constexpr size_t lds = ring_lds_bytes<FMT, DUAL, MT, NS, WV>();
+    constexpr int BM = 32 * MT * WM, BNO = (DUAL ? 32 : 64) * WN;
+    constexpr size_t lds = ring_lds_bytes<FMT, MT, WM, WN, NS>();
     static bool attr_set = false;
     if (!attr_set) {
-        CHIP_CHECK(hipFuncSetAttribute((const void *)gemm_ring_kernel<FMT, DUAL, MT, NS, WV>,
+        CHIP_CHECK(hipFuncSetAttribute((const void *)gemm_ring_kernel<FMT, DUAL, MT, WM, WN, NS, QG>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         attr_set = true;
     }
-    const dim3 grid((a.N + BN - 1) / BN * ((a.M + BM - 1) / BM), 1, split ? a.nstored : 1);
-    hipLaunchKernelGGL((gemm_ring_kernel<FMT, DUAL, MT, NS, WV>), grid, dim3(64 * WV), lds, s, a, split);
+    const dim3 grid((a.N + BNO - 1) / BNO * ((a.M + BM - 1) / BM), 1, split ? a.nstored : 1);
+    hipLaunchKernelGGL((gemm_ring_kernel<FMT, DUAL, MT, WM, WN, NS, QG>), grid, dim3(64 * WM * WN), lds, s, a, split);
     CHIP_CHECK(hipGetLastError());
     if (split && !a.defer) {
         const size_t MN = (size_t)a.M * a.N;
@@ -862,69 +872,111 @@ int launch_mt(const GArgs &a, bool split, hipStream_t s) {
     return 0;
 }
 
-// Whether `blocks` blocks of one per CU keep at least 3/4 of the CU slots of
-// their rounds busy (288 blocks on 256 CUs: a second round of 32 does not).
-bool fills_rounds(long blocks, long cus) {
-    const long rounds = (blocks + cus - 1) / cus;
-    return blocks >= 1 && 4 * blocks >= 3 * rounds * cus;
+// Ring stages by format: the 4-wave tile keeps two blocks per CU (64 to 76 KB
+// each), the others one.
+template <int FMT>
+constexpr int ring_stages() { return FMT == FMT_BF16 ? 4 : 5; }
+
+enum Tile : int { TILE_64x128, TILE_128x128, TILE_128x256 };
+// How a ring GEMM runs: its tile and its K split (0 none, 1 per chunk, 2 a
+// single matrix's two halves) with the sums stored per output.
+struct RingPlan {
+    int tile, split, nstored;
+    size_t ws_floats;
+};
+
+// The plan with the least estimated time of those whose stored sums fit
+// ws_floats. The estimate, in us: rounds of the tile's blocks (one per CU, two
+// for the 4-wave tile) times the time of 1,024 columns of a block in a full
+// round (with no more blocks than CUs, of a block alone), and 3 to fill and
+// drain; a split adds a launch or a longer reader (2) and its sums' write and
+// read at 4.5 TB/s. Measured per 1,024 columns: 128 x 256 tiles 31 us (BF16)
+// and 34 (Q8/Q4) on 256 CUs, 128 x 128 18 to 20, 64 x 128 24 (27), alone 16
+// (18 to 20). Examples (BF16, x split included), chosen against the next best:
+// 14336 x 4096 at 512 tokens 128 x 256 unsplit 119 us (128 x 128 152); 4096 x
+// 14336 at 512 128 x 128 halves 152 (128 x 256 halves 175); 6144 x 4096 at 512
+// 128 x 256 halves 69 (128 x 128 unsplit 78); 4096 x 4096 at 256 128 x 128
+// halves 45 (64 x 128 per chunk 60), at 192 64 x 128 halves 39 (128 x 128
+// halves 41); 1152 x 896 at 128 64 x 128 per chunk 11.9 (128 x 128 13.0); 3584
+// x 18944 at 128 128 x 128 per chunk 67 (64 x 128 80).
+RingPlan ring_plan(int fmt, bool dual, int N, int K, int M, size_t ws_floats) {
+    static constexpr struct {
+        int bm, bn, per_cu;
+        float us_bf16, us_quant;    // a full round
+        float low_bf16, low_quant;  // no more blocks than CUs
+    } kTiles[] = {{64, 128, 2, 24.f, 27.f, 16.f, 19.f},
+                  {128, 128, 1, 19.f, 19.f, 19.f, 19.f},
+                  {128, 256, 1, 30.f, 34.f, 30.f, 34.f}};
+    const int chunk = gemm_chunk_depth(K), nchunks = (K + chunk - 1) / chunk;
+    const long cus = device_cus();
+    const float mn = (float)M * (float)N;
+    RingPlan best{TILE_128x128, 0, 1, 0};
+    float best_us = 0.f;
+    for (int t = 0; t < 3; ++t) {
+        const int bno = dual ? kTiles[t].bn / 2 : kTiles[t].bn;
+        const long tiles = (long)((N + bno - 1) / bno) * ((M + kTiles[t].bm - 1) / kTiles[t].bm);
+        const bool bf = fmt == FMT_BF16;
+        for (int split = 0; split < 3; ++split) {
+            if (split && (nchunks == 1 || (split == 2 && dual))) continue;
+            const int parts = split == 1 ? nchunks : split == 2 ? 2 : 1;
+            const int depth = split == 1 ? chunk : split == 2 ? (nchunks + 1) / 2 * chunk : K;
+            const size_t need = split ? (size_t)parts * M * N * (dual ? 2 : 1) : 0;
+            if (need > ws_floats) continue;
+            const long slots = cus * kTiles[t].per_cu, rounds = (tiles * parts + slots - 1) / slots;
+            const float us = tiles * parts > cus ? bf ? kTiles[t].us_bf16 : kTiles[t].us_quant
+                                                 : bf ? kTiles[t].low_bf16 : kTiles[t].low_quant;
+            float est = (float)rounds * (float)depth / 1024.f * us + 3.f;
+            if (split) est += 2.f + 8.f * (float)parts * (dual ? 2.f : 1.f) * mn / 4.5e6f;
+            if (best_us == 0.f || est < best_us) {
+                best_us = est;
+                best = RingPlan{t, split, parts, need};
+            }
+        }
+    }
+    return best;
 }
-// 8-wave blocks of 128 tokens x 128 rows: their tiles cover at least 7/8 of
-// the CUs and fill their rounds.
-bool gemm_w8(int N, int M) {
-    const long tiles128 = (long)((N + BN - 1) / BN) * ((M + 127) / 128), cus = device_cus();
-    return tiles128 * 8 >= cus * 7 && fills_rounds(tiles128, cus);
-}
-// Whether a single matrix's GEMM runs as two chunk halves on 8-wave blocks:
-// two blocks per 128-token tile fill 95-100 % of the CUs in one round, and
-// it has more than one chunk.
-bool gemm_halves_split(int N, int M, int nchunks) {
-    const long tiles128 = (long)((N + BN - 1) / BN) * ((M + 127) / 128), cus = device_cus();
-    return nchunks > 1 && 2 * tiles128 * 20 >= cus * 19 && 2 * tiles128 <= cus;
+
+template <int FMT, bool DUAL, int QG>
+int launch_ring_plan(GArgs &a, const RingPlan &p, hipStream_t s) {
+    constexpr int NS = ring_stages<FMT>();
+    a.nstored = p.nstored;
+    switch (p.tile) {
+        case TILE_64x128: return launch_ring<FMT, DUAL, 1, 2, 2, NS, QG>(a, p.split, s);
+        case TILE_128x128: return launch_ring<FMT, DUAL, 1, 4, 2, NS, QG>(a, p.split, s);
+        default: return launch_ring<FMT, DUAL, 2, 2, 4, NS, QG>(a, p.split, s);
+    }
 }
 
 template <int FMT>
 int launch_fmt(GArgs a, bool dual, size_t ws_floats, hipStream_t s, bool &split_out, int &stored_out) {
+    // Pre-split x with K a multiple of the stage and 32-bit buffer offsets:
+    // the ring kernel (weights copied 16 bytes at a time, Q4 and unaligned Q8 4).
+    const int galign = FMT == FMT_BF16 ? 16 : 4;
+    const bool ring = a.xh && a.K % BK == 0 && a.stride % galign == 0 &&
+                      ((uintptr_t)a.w % galign) == 0 &&
+                      (!dual || (((uintptr_t)a.w | (uintptr_t)a.w2 | a.stride) % (FMT == FMT_Q4 ? 4 : 16)) == 0) &&
+                      (size_t)a.M * a.K * 2 < (1ull << 31) && (size_t)a.N * a.stride < (1ull << 31);
+    if (ring) {
+        const RingPlan p = ring_plan(FMT, dual, a.N, a.K, a.M, a.ws ? ws_floats : 0);
+        split_out = p.split != 0;
+        stored_out = p.nstored;
+        if constexpr (FMT == FMT_Q8) {  // a single matrix of odd row count
+            if (!dual && ((uintptr_t)a.w % 16 || a.stride % 16)) return launch_ring_plan<FMT, false, 4>(a, p, s);
+        }
+        return dual ? launch_ring_plan<FMT, true, 16>(a, p, s) : launch_ring_plan<FMT, false, 16>(a, p, s);
+    }
+    // Otherwise (K not a multiple of the stage, x not pre-split, or operands
+    // beyond the buffer loads' 32-bit offsets): the register-staged kernel.
+    // Many tiles: fold in registers. Few tiles: split-K over the chunks when
+    // the workspace holds them.
     const long n_tiles = (a.N + BN - 1) / BN;
     const long tiles128 = n_tiles * ((a.M + 127) / 128), tiles64 = n_tiles * ((a.M + 63) / 64);
     const long cus = device_cus();
-    // Many tiles: fold in registers. Few tiles: split-K over the chunks when
-    // the workspace holds them.
     const bool split = a.nchunks > 1 && tiles64 < cus && a.ws &&
-                       ws_floats >= gemm_workspace_floats(a.N, a.K, a.M, dual);
+                       ws_floats >= (size_t)a.nchunks * a.M * a.N * (dual ? 2 : 1);
     split_out = split;
     a.nstored = a.nchunks;
     stored_out = a.nstored;
-    // Pre-split x with K a multiple of the stage and 32-bit buffer offsets:
-    // the ring kernel (weights copied 16 bytes at a time, Q4 4 at a time).
-    const int galign = FMT == FMT_Q4 ? 4 : 16;
-    const bool ring = a.xh && a.K % BK == 0 && a.stride % galign == 0 &&
-                      ((uintptr_t)a.w % galign) == 0 && (!dual || ((uintptr_t)a.w2 % galign) == 0) &&
-                      (size_t)a.M * a.K * 2 < (1ull << 31) && (size_t)a.N * a.stride < (1ull << 31);
-    // 8-wave blocks of 128 tokens x 128 rows where those tiles cover at
-    // least 7/8 of the CUs: each converted weight tile and each x tile in
-    // LDS then serves twice the MFMAs of a 4-wave 64-token block, with the
-    // same waves per CU (one 8-wave block against two 4-wave ones). Measured
-    // at 1,024 tokens: BF16 4096x4096 358 -> 418, 4096x14336 310 -> 402,
-    // 3584x18944 298 -> 370 TFLOP/s; Llama-3-8B Q4 512-row prefill 17.2K ->
-    // 18.6K tok/s (mostly the dual gate/up, which before took 128-token tiles
-    // on 4 waves), Qwen2-7B 1,024-row 18.2K -> 19.2K; the same bits. Where
-    // the 128-token tiles cover only half the CUs (4096 rows at 512 tokens:
-    // 128 tiles), 4-wave 64-token blocks are faster (307 vs 242 TFLOP/s).
-    if (ring && !split && gemm_w8(a.N, a.M))
-        return dual ? launch_ring<FMT, true, 1, 8>(a, 0, s) : launch_ring<FMT, false, 1, 8>(a, 0, s);
-    // A single matrix whose 128-token tiles cover half the CUs (4,096 rows
-    // at 512 tokens: 128 tiles): its two chunk halves on separate 8-wave
-    // blocks, the half sums folded by the reader.
-    if (ring && !split && !dual && gemm_halves_split(a.N, a.M, a.nchunks) && a.ws &&
-        ws_floats >= 2 * (size_t)a.M * a.N) {
-        split_out = true;
-        a.nstored = stored_out = 2;
-        return launch_ring<FMT, false, 1, 8>(a, 2, s);
-    }
-    const int sp = split ? 1 : 0;
-    if (ring) return dual ? launch_ring<FMT, true, 1>(a, sp, s) : launch_ring<FMT, false, 1>(a, sp, s);
-    // Otherwise (K not a multiple of the stage, x not pre-split, or operands
-    // beyond the buffer loads' 32-bit offsets): the register-staged kernel.
     if (dual) return launch_mt<FMT, true, 1>(a, split, s);
     if (!split && tiles128 >= cus) return launch_mt<FMT, false, 2>(a, false, s);
     return launch_mt<FMT, false, 1>(a, split, s);
@@ -978,23 +1030,19 @@ int gemm_chunk_depth(int K) {
     return (want + BK - 1) / BK * BK;
 }
 
-size_t gemm_workspace_floats(size_t N, size_t K, size_t M, bool dual) {
+size_t gemm_workspace_floats(int fmt, size_t N, size_t K, size_t M, bool dual) {
+    if (std::max({N, K, M}) > (size_t)INT32_MAX) return 0;  // launch_gemm refuses it
+    // The register-staged kernel (unaligned operands, other K) splits per
+    // chunk while 64-token tiles leave CUs idle.
     const int chunk = gemm_chunk_depth((int)K);
-    const size_t nchunks = (K + chunk - 1) / chunk;
-    if (nchunks <= 1) return 0;
-    return nchunks * M * N * (dual ? 2 : 1);
+    const size_t nchunks = (K + chunk - 1) / chunk, tiles = (N + BN - 1) / BN * ((M + 63) / 64);
+    const size_t staged = nchunks > 1 && tiles < (size_t)device_cus() ? nchunks * M * N * (dual ? 2 : 1) : 0;
+    return K % BK ? staged : std::max(staged, ring_plan(fmt, dual, (int)N, (int)K, (int)M, SIZE_MAX).ws_floats);
 }
 
-size_t gemm_split_workspace_floats(size_t N, size_t K, size_t m_max, bool dual) {
-    // The per-chunk split runs only while 64-token tiles leave CUs idle; the
-    // two-half split (single matrices) while two blocks per 128-token tile
-    // fit the CUs once.
-    const size_t n_tiles = (N + BN - 1) / BN, cus = (size_t)device_cus();
-    const size_t m_split = 64 * ((cus + n_tiles - 1) / n_tiles);
-    size_t need = gemm_workspace_floats(N, K, std::min(m_max, m_split), dual);
-    const int chunk = gemm_chunk_depth((int)K);
-    if (!dual && (K + chunk - 1) / chunk > 1)
-        need = std::max(need, 2 * std::min(m_max, 128 * (cus / (2 * n_tiles))) * N);
+size_t gemm_split_workspace_floats(int fmt, size_t N, size_t K, size_t m_max, bool dual) {
+    size_t need = gemm_workspace_floats(fmt, N, K, m_max, dual);
+    for (size_t m = 64; m < m_max; m += 64) need = std::max(need, gemm_workspace_floats(fmt, N, K, m, dual));
     return need;
 }
 

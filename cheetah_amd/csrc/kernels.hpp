@@ -73,9 +73,11 @@ struct GemmJob {
 int launch_gemm(const GemmJob &job, hipStream_t stream);
 int launch_split_bf16(const float *x, size_t n, uint16_t *xh, uint16_t *xl, hipStream_t s);
 int gemm_chunk_depth(int K);
-size_t gemm_workspace_floats(size_t N, size_t K, size_t M, bool dual);
-// Scratch the split path can use for any token count up to m_max.
-size_t gemm_split_workspace_floats(size_t N, size_t K, size_t m_max, bool dual);
+// Split-K scratch a GEMM of M tokens uses; with less it runs another split
+// or none (the same bits).
+size_t gemm_workspace_floats(int fmt, size_t N, size_t K, size_t M, bool dual);
+// The same for any token count up to m_max.
+size_t gemm_split_workspace_floats(int fmt, size_t N, size_t K, size_t m_max, bool dual);
 
 // ---------------------------------------------------------------------------
 // Quantization (bit-exact to q8.rs / q4.rs quantize) and dequantization.

@@ -678,10 +678,11 @@ int init_instance(cheetah_hip_model *m) {
     CHIP_TRY(m->mem.alloc(&m->part, m->part_floats));
     {
         const size_t qd = sh.q_dim(), kvd = sh.kv_dim(), I = c.intermediate_size, H = c.hidden_size;
-        m->gemm_ws_floats = std::max({gemm_split_workspace_floats(qd + 2 * kvd, H, R, false),
-                                      gemm_split_workspace_floats(H, qd, R, false),
-                                      gemm_split_workspace_floats(I, H, R, true),
-                                      gemm_split_workspace_floats(H, I, R, false), (size_t)1});
+        const int fmt = sh.layers[0].qkv.fmt;
+        m->gemm_ws_floats = std::max({gemm_split_workspace_floats(fmt, qd + 2 * kvd, H, R, false),
+                                      gemm_split_workspace_floats(fmt, H, qd, R, false),
+                                      gemm_split_workspace_floats(fmt, I, H, R, true),
+                                      gemm_split_workspace_floats(fmt, H, I, R, false), (size_t)1});
         CHIP_TRY(m->mem.alloc(&m->gemm_ws, m->gemm_ws_floats));
         const size_t width = std::max({H, qd, I});
         CHIP_TRY(m->mem.alloc(&m->xh, R * width));

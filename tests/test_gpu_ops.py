@@ -159,6 +159,32 @@ def test_gemm_bits_independent_of_token_count(hip, fmt):
     assert np.isfinite(y1024).all() and np.abs(y1024).max() > 0
 
 
+@pytest.mark.parametrize("fmt", ["bf16", "q8", "q4"])
+@pytest.mark.parametrize("rows,cols", [(1001, 64), (515, 896), (4097, 4096), (14336, 1024)])
+def test_gemm_tile_edges_give_the_same_bits(hip, oracle, fmt, rows, cols):
+    """Token counts and row counts around the edges of the 64 / 128-token and
+    128 / 256-row tiles, odd row counts (Q8 payloads only 4-byte aligned) and
+    every K split the sizes choose: a token's outputs are the same bits in
+    every call, and the oracle's within the hi/lo input split (2^-17 per
+    product; 1e-5 of the largest output)."""
+    rng = np.random.default_rng(rows + cols)
+    x = rng.standard_normal((1030, cols)).astype(np.float32)
+    if fmt == "bf16":
+        w = synth.f32_to_bf16(rng.standard_normal((rows, cols)).astype(np.float32))
+        wd = hip.DeviceBuffer.from_array(w)
+    else:
+        buf = random_quant(rng, fmt, rows, cols)
+        wd = hip.DeviceBuffer.from_array(buf)
+    full = np.ascontiguousarray(hip.gemm(wd, fmt, rows, cols, x))
+    for n in (1, 63, 64, 65, 128, 129, 257, 389, 512):
+        got = np.ascontiguousarray(hip.gemm(wd, fmt, rows, cols, x[:n]))
+        assert np.array_equal(got.view(np.uint32), full[:n].view(np.uint32)), n
+    sel = np.array([0, 63, 64, 127, 128, 1023, 1024, 1029])
+    xs = np.ascontiguousarray(x[sel])
+    ref = oracle.gemm_bf16(w, xs) if fmt == "bf16" else oracle.gemm_quant(buf, rows, cols, xs, fmt)
+    assert rel_err(full[sel], ref) < 1e-5
+
+
 def _attn_case(rng, q_heads, kv_heads, hd, ctx, rows):
     k = synth.f32_to_bf16(rng.standard_normal((ctx, kv_heads, hd)).astype(np.float32))
     v = synth.f32_to_bf16(rng.standard_normal((ctx, kv_heads, hd)).astype(np.float32))
