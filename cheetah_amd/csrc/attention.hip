@@ -708,7 +708,17 @@ __global__ __launch_bounds__(kThreads) void attn_combine_kernel(const float *par
 // K rows are staged in LDS with bits 2 and 3 of the position swapped, which
 // makes the S^T output registers exactly the B operand layout of the second
 // product (8 consecutive positions per lane), so P never moves between lanes.
-// V is staged transposed ([dim][position]).
+// V rows are staged as they come and read transposed (ds_read_b64_tr_b16).
+//
+// Bound: the matrix cores at two waves per SIMD (236 registers at head_dim
+// 128). Both tiles' copies go global -> LDS by buffer loads and the LDS reads
+// are such that the compiler waits for no copy in flight: with global loads to
+// LDS, builtin transposing reads or a vector load of the page table it waited
+// for the next tile's copies (or the table) inside every tile. V through
+// registers and 16-bit transposing stores cost the rest. 512 rows on a 4K
+// prefix, 32 q / 8 KV heads of 128: 113 -> 89.8 us (316 -> 398 TFLOP/s, twice
+// that executed), with the same bits; rows direct to LDS and transposing reads
+// alone 97.5 us.
 //
 // Splits are absolute position ranges of `span` keys (fixed per model), so
 // every row's result depends only on its own position (the same bits however
@@ -770,16 +780,59 @@ __device__ __forceinline__ void store_prefill_rows(const AttnArgs &a, const f32x
     }
 }
 
+// Chunk swizzle of V row r: the rows a transposing read takes together (four
+// consecutive ones, 64 bytes each) fall on distinct banks, and rows r and
+// r + 4 share it.
+template <int HD>
+__device__ __forceinline__ int vseg(int r) {
+    return HD == 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1);
+}
+
+// The V^T fragments of 16 positions, all HD dims, by transposing LDS reads at
+// the UT lane addresses + OFF (rows 0..3) and + OFF + 4 rows. Inline assembly:
+// for the builtin the compiler waits for every copy in flight (the next tile's)
+// first; each block waits for its own data.
+template <int HD, int OFF>
+__device__ __forceinline__ void read_vt(const uint32_t (&addr)[HD / 32], bf16x8 (&va)[HD / 32]) {
+    constexpr int OFF4 = OFF + 4 * HD * 2;
+    s16x4_t r[HD / 32][2];
+    if constexpr (HD == 128) {
+        asm volatile(
+            "ds_read_b64_tr_b16 %0, %8 offset:%12\n\tds_read_b64_tr_b16 %1, %8 offset:%13\n\t"
+            "ds_read_b64_tr_b16 %2, %9 offset:%12\n\tds_read_b64_tr_b16 %3, %9 offset:%13\n\t"
+            "ds_read_b64_tr_b16 %4, %10 offset:%12\n\tds_read_b64_tr_b16 %5, %10 offset:%13\n\t"
+            "ds_read_b64_tr_b16 %6, %11 offset:%12\n\tds_read_b64_tr_b16 %7, %11 offset:%13\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(r[0][0]), "=&v"(r[0][1]), "=&v"(r[1][0]), "=&v"(r[1][1]), "=&v"(r[2][0]), "=&v"(r[2][1]),
+              "=&v"(r[3][0]), "=&v"(r[3][1])
+            : "v"(addr[0]), "v"(addr[1]), "v"(addr[2]), "v"(addr[3]), "i"(OFF), "i"(OFF4)
+            : "memory");
+    } else {
+        asm volatile(
+            "ds_read_b64_tr_b16 %0, %4 offset:%6\n\tds_read_b64_tr_b16 %1, %4 offset:%7\n\t"
+            "ds_read_b64_tr_b16 %2, %5 offset:%6\n\tds_read_b64_tr_b16 %3, %5 offset:%7\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(r[0][0]), "=&v"(r[0][1]), "=&v"(r[1][0]), "=&v"(r[1][1])
+            : "v"(addr[0]), "v"(addr[1]), "i"(OFF), "i"(OFF4)
+            : "memory");
+    }
+#pragma unroll
+    for (int u = 0; u < HD / 32; ++u)
+        va[u] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(r[u][0], r[u][1], 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 template <int HD, int G>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill_kernel(AttnArgs a, int rows, int S, int span) {
     constexpr int RW = 32 / G, MV = RW * G;
-    constexpr int LDV = 64 + 8;
     constexpr int KSTEPS = HD / 16, UT = HD / 32, KC = HD / 32;
     constexpr int CPR = HD / 8;  // 16-byte chunks per K row
-    // K rows unpadded, chunk c of LDS row r stored at chunk c ^ (r % CPR).
-    __shared__ __attribute__((aligned(16))) uint16_t ks[2][64 * HD];
-    __shared__ __attribute__((aligned(16))) uint16_t vt[2][HD * LDV];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // Two tiles each. K rows unpadded, chunk c of LDS row r stored at chunk
+    // c ^ (r % CPR); V rows as they come, 64-byte segments swizzled by vseg.
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem_kv[];
+    uint8_t *ks = smem_kv, *vs = smem_kv + 2 * 64 * HD * 2;
+    constexpr int TB = 64 * HD * 2;  // bytes of one tile
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int n = lane & 31, half = lane >> 5;
     const int rb = blockIdx.x, g = blockIdx.y, split = blockIdx.z;
     const int row = rb * 4 * RW + wave * RW + n / G;
@@ -803,87 +856,102 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     bf16x8 qh[KSTEPS], ql[KSTEPS];
     {
         const float sl2 = (1.0f / sqrtf((float)HD)) * 1.44269504088896340736f;
-        const float *qp = a.q + (size_t)(rvalid ? row : 0) * a.q_stride + (size_t)head * HD + 8 * half;
+        const float *qp = a.q + (size_t)(rvalid ? row : 0) * a.q_stride + (size_t)(rvalid ? head : 0) * HD + 8 * half;
+        const float sq = rvalid ? sl2 : 0.f;  // rows without a query: their scores are not used
+        f32x4 raw[KSTEPS][2];  // every load before the first use: one round trip
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s) {
-            float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            if (rvalid) {
-                const f32x4 t0 = *(const f32x4 *)(qp + 16 * s), t1 = *(const f32x4 *)(qp + 16 * s + 4);
-                v[0] = t0[0] * sl2; v[1] = t0[1] * sl2; v[2] = t0[2] * sl2; v[3] = t0[3] * sl2;
-                v[4] = t1[0] * sl2; v[5] = t1[1] * sl2; v[6] = t1[2] * sl2; v[7] = t1[3] * sl2;
-            }
+            raw[s][0] = *(const f32x4 *)(qp + 16 * s);
+            raw[s][1] = *(const f32x4 *)(qp + 16 * s + 4);
+        }
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+            const float v[8] = {raw[s][0][0] * sq, raw[s][0][1] * sq, raw[s][0][2] * sq, raw[s][0][3] * sq,
+                                raw[s][1][0] * sq, raw[s][1][1] * sq, raw[s][1][2] * sq, raw[s][1][3] * sq};
             split8(v, qh[s], ql[s]);
         }
     }
 
-    const uint16_t *kbase = (const uint16_t *)a.k, *vbase = (const uint16_t *)a.v;
-    u32x4 vr[KC];
-    // K: direct global->LDS copies. One wave instruction fills 1 KB = 64 / CPR
-    // LDS rows; lane i lands at byte 16 i, so it fetches the global chunk
-    // that the swizzle places there. Rows past the split end may hold stale
-    // bytes: their scores are masked before use.
-    auto fetch_k = [&](int t0, int b) {
-        const int page = a.page_table[t0 / a.page_size];
+    // K and V: direct global->LDS copies (buffer loads: the compiler waits for
+    // no copy in flight when it reads LDS). Copy c of a wave fills 1 KB =
+    // 64 / CPR LDS rows from row r0 = (wave + 4 c) 64 / CPR on; lane i lands at
+    // byte 16 i, so it fetches the global chunk that the swizzle places there.
+    // c moves r0 by a multiple of 16: the lane's offset is the same plus 4 KB.
+    // K rows past the split end may hold stale bytes: their scores are masked
+    // before use.
+    constexpr int RPI = 64 / CPR;
+    const int lr = wave * RPI + lane / CPR;  // LDS row of copy 0
+    const int koff = krow_of(lr) * HD * 2 + 16 * ((lane % CPR) ^ (lr % CPR));
+    const int voff = lr * HD * 2 + 16 * ((lane % CPR) ^ vseg<HD>(lr));
+    // Page of the tile at t0: a scalar load, one tile ahead of its use.
+    auto page_of = [&](int t0) {
+        return ((const __attribute__((address_space(4))) int32_t *)a.page_table)[t0 / a.page_size];
+    };
+    auto fetch = [&](int t0, int page, int b) {
         const size_t tile = (((size_t)page * a.kv_heads + g) * a.page_size + (t0 % a.page_size)) * HD;
-        constexpr int RPI = 64 / CPR;  // LDS rows per wave instruction
+        const __amdgpu_buffer_rsrc_t rk =
+            __builtin_amdgcn_make_buffer_rsrc((void *)((const uint16_t *)a.k + tile), (short)0, TB, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rv =
+            __builtin_amdgcn_make_buffer_rsrc((void *)((const uint16_t *)a.v + tile), (short)0, TB, 0x00020000);
 #pragma unroll
-        for (int c = 0; c < KC; ++c) {
-            const int r0 = (wave + 4 * c) * RPI;  // first LDS row of this instruction
-            const int r = r0 + lane / CPR, cs = lane % CPR;
-            const int p = krow_of(r), chunk = cs ^ (r % CPR);
-            __builtin_amdgcn_global_load_lds(kbase + tile + (size_t)p * HD + chunk * 8,
-                                             (__attribute__((address_space(3))) void *)(&ks[b][r0 * HD]), 16, 0, 0);
-        }
+        for (int c = 0; c < KC; ++c) buf_to_lds<16>(rk, ks + b * TB + wave * 1024 + 4096 * c, koff, 4096 * c);
+#pragma unroll
+        for (int c = 0; c < KC; ++c) buf_to_lds<16>(rv, vs + b * TB + wave * 1024 + 4096 * c, voff, 4096 * c);
     };
-    auto fetch_v = [&](int t0) {
-        const int page = a.page_table[t0 / a.page_size];
-        const size_t tile = (((size_t)page * a.kv_heads + g) * a.page_size + (t0 % a.page_size)) * HD;
+    // This wave's V rows past the split end, once they have landed: they may
+    // be unwritten memory, and a probability of 0 does not clear a NaN.
+    auto clear_v = [&](int t0, int b) {
 #pragma unroll
-        for (int c = 0; c < KC; ++c) {
-            const int idx = tid + kThreads * c, p = idx / CPR, d0 = (idx % CPR) * 8;
-            // positions past the split end may be unwritten: zeros (p = 0 there)
-            vr[c] = t0 + p < end ? *(const u32x4 *)(vbase + tile + p * HD + d0) : u32x4{0u, 0u, 0u, 0u};
-        }
+        for (int c = 0; c < KC; ++c)
+            if (t0 + lr + 4 * RPI * c >= end)
+                *(u32x4 *)(vs + b * TB + wave * 1024 + 4096 * c + 16 * lane) = u32x4{0u, 0u, 0u, 0u};
     };
-    auto store_v = [&](int b) {
+    // This lane's transposing V reads in a 16-position block: rows
+    // 8 half + i / 4 (and + 4), dims 32 u + 16 ((lane / 16) % 2) + 4 (i % 4).
+    const int vi = lane & 15, vrow = 8 * half + (vi >> 2);
+    uint32_t vaddr[UT];
 #pragma unroll
-        for (int c = 0; c < KC; ++c) {
-            const int idx = tid + kThreads * c, p = idx / CPR, d0 = (idx % CPR) * 8;
-            const int col = vcol(d0, p);
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                vt[b][(d0 + e) * LDV + col] = (uint16_t)((e & 1) ? (vr[c][e >> 1] >> 16) : (vr[c][e >> 1] & 0xFFFFu));
-        }
-    };
+    for (int u = 0; u < UT; ++u) {
+        const int chunk = (4 * u + 2 * ((lane >> 4) & 1) + ((vi & 3) >> 1)) ^ vseg<HD>(vrow);
+        vaddr[u] = (uint32_t)(uintptr_t)(vs + vrow * HD * 2 + 16 * chunk + 8 * (vi & 1));
+    }
 
     f32x16 oacc[UT];
 #pragma unroll
     for (int u = 0; u < UT; ++u) oacc[u] = f32x16{};
     float m2 = -INFINITY, l = 0.f;
-    fetch_k(start, 0);
-    fetch_v(start);
-    store_v(0);
+    fetch(start, page_of(start), 0);
+    const int last_tile = start + (end - 1 - start) / 64 * 64;
+    int page_next = page_of(min(start + 64, last_tile));
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (start + 64 > end) clear_v(start, 0);
     __syncthreads();
     int b = 0;
     for (int t0 = start; t0 < end; t0 += 64) {
         const bool more = t0 + 64 < end;
         if (more) {
-            fetch_k(t0 + 64, b ^ 1);
-            fetch_v(t0 + 64);
+            fetch(t0 + 64, page_next, b ^ 1);
+            page_next = page_of(min(t0 + 128, last_tile));
         }
         // Two halves of 32 positions, each: S^T, online softmax, O^T update.
+        uint32_t vad[UT];
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
+        for (int u = 0; u < UT; ++u) vad[u] = vaddr[u] + b * TB;
+        auto half_tile = [&](auto half_index) {
+            constexpr int tt = decltype(half_index)::value;
             f32x16 sacc = f32x16{};
 #pragma unroll
             for (int s = 0; s < KSTEPS; ++s) {
                 const int r = 32 * tt + n;
                 const bf16x8 ka =
-                    __builtin_bit_cast(bf16x8, *(const u32x4 *)(&ks[b][r * HD + (((2 * s + half) ^ (r % CPR)) << 3)]));
+                    __builtin_bit_cast(bf16x8, *(const u32x4 *)(ks + b * TB + r * HD * 2 + 16 * ((2 * s + half) ^ (r % CPR))));
                 sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, qh[s], sacc, 0, 0, 0);
                 sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, ql[s], sacc, 0, 0, 0);
             }
+            // The half's V^T fragments, while the score products drain.
+            bf16x8 va[2][UT];
+            read_vt<HD, (32 * tt) * HD * 2>(vad, va[0]);
+            read_vt<HD, (32 * tt + 16) * HD * 2>(vad, va[1]);
             // Causal / split-end mask, only where the half reaches past a
             // row's position or past the split (block-uniform test).
             const int h0 = t0 + 32 * tt;
@@ -934,16 +1002,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
                 split8(pv, bh, bl);
 #pragma unroll
                 for (int u = 0; u < UT; ++u) {
-                    const int d = 32 * u + n;
-                    const bf16x8 va = __builtin_bit_cast(
-                        bf16x8, *(const u32x4 *)(&vt[b][d * LDV + vcol(d, 32 * tt + 16 * s2 + 8 * half)]));
-                    oacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, bh, oacc[u], 0, 0, 0);
-                    oacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, bl, oacc[u], 0, 0, 0);
+                    oacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[s2][u], bh, oacc[u], 0, 0, 0);
+                    oacc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[s2][u], bl, oacc[u], 0, 0, 0);
                 }
             }
-        }
-        if (more) store_v(b ^ 1);
+        };
+        half_tile(std::integral_constant<int, 0>{});
+        half_tile(std::integral_constant<int, 1>{});
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (more && t0 + 128 > end) clear_v(t0 + 64, b ^ 1);
         __syncthreads();
         b ^= 1;
     }
@@ -1039,8 +1106,10 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
     // V unit: 4 dims of positions 4 (idx / (HD / 4)) .. + 3.
     const float *kbase = (const float *)a.k, *vbase = (const float *)a.v;
     f32x4 kr[KU][2], vr[VU][4];
-    auto fetch = [&](int t0) {
-        const int page = a.page_table[t0 / a.page_size];
+    auto page_of = [&](int t0) {  // a scalar load, one tile ahead of its use
+        return ((const __attribute__((address_space(4))) int32_t *)a.page_table)[t0 / a.page_size];
+    };
+    auto fetch = [&](int t0, int page) {
         const size_t tile = (((size_t)page * a.kv_heads + g) * a.page_size + (t0 % a.page_size)) * HD;
 #pragma unroll
         for (int c = 0; c < KU; ++c) {
@@ -1083,21 +1152,26 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
             }
         }
     };
-    fetch(start);
+    fetch(start, page_of(start));
+    const int last_tile = start + (end - 1 - start) / 64 * 64;
+    int page_next = page_of(min(start + 64, last_tile));
 
     // Q^T operands, pre-scaled by log2(e) / sqrt(HD) (scores in the exp2 domain).
     bf16x8 q3[KSTEPS][3];
     {
         const float sl2 = (1.0f / sqrtf((float)HD)) * 1.44269504088896340736f;
-        const float *qp = a.q + (size_t)(rvalid ? row : 0) * a.q_stride + (size_t)head * HD + 8 * half;
+        const float *qp = a.q + (size_t)(rvalid ? row : 0) * a.q_stride + (size_t)(rvalid ? head : 0) * HD + 8 * half;
+        const float sq = rvalid ? sl2 : 0.f;  // rows without a query: their scores are not used
+        f32x4 raw[KSTEPS][2];  // every load before the first use: one round trip
 #pragma unroll
         for (int s = 0; s < KSTEPS; ++s) {
-            float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            if (rvalid) {
-                const f32x4 t0 = *(const f32x4 *)(qp + 16 * s), t1 = *(const f32x4 *)(qp + 16 * s + 4);
-                v[0] = t0[0] * sl2; v[1] = t0[1] * sl2; v[2] = t0[2] * sl2; v[3] = t0[3] * sl2;
-                v[4] = t1[0] * sl2; v[5] = t1[1] * sl2; v[6] = t1[2] * sl2; v[7] = t1[3] * sl2;
-            }
+            raw[s][0] = *(const f32x4 *)(qp + 16 * s);
+            raw[s][1] = *(const f32x4 *)(qp + 16 * s + 4);
+        }
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+            const float v[8] = {raw[s][0][0] * sq, raw[s][0][1] * sq, raw[s][0][2] * sq, raw[s][0][3] * sq,
+                                raw[s][1][0] * sq, raw[s][1][1] * sq, raw[s][1][2] * sq, raw[s][1][3] * sq};
             split3x8(v, q3[s]);
         }
     }
@@ -1110,7 +1184,10 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
         __syncthreads();  // the previous tile's reads are done
         stage();
         __syncthreads();
-        if (t0 + 64 < end) fetch(t0 + 64);
+        if (t0 + 64 < end) {
+            fetch(t0 + 64, page_next);
+            page_next = page_of(min(t0 + 128, last_tile));
+        }
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt) {
             f32x16 sacc = f32x16{}, slow = f32x16{};
@@ -1245,7 +1322,14 @@ int launch_prefill_hg(const AttnJob &j, const AttnArgs &a, int S, hipStream_t s)
         hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, G>), dim3(rb, j.g.kv_heads, S), dim3(kThreads), lds, s, a,
                            (int)j.rows, S, j.span);
     } else {
-        hipLaunchKernelGGL((attn_prefill_kernel<HD, G>), dim3(rb, j.g.kv_heads, S), dim3(kThreads), 0, s, a,
+        constexpr size_t lds = (size_t)4 * 64 * HD * 2;
+        static bool attr_set = false;
+        if (!attr_set) {
+            CHIP_CHECK(hipFuncSetAttribute((const void *)attn_prefill_kernel<HD, G>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            attr_set = true;
+        }
+        hipLaunchKernelGGL((attn_prefill_kernel<HD, G>), dim3(rb, j.g.kv_heads, S), dim3(kThreads), lds, s, a,
                            (int)j.rows, S, j.span);
     }
     CHIP_CHECK(hipGetLastError());

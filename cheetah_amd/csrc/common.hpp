@@ -142,4 +142,14 @@ __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(fmaxf(lane_read(v, 0), lane_read(v, 16)), fmaxf(lane_read(v, 32), lane_read(v, 48)));
 }
 
+typedef __attribute__((address_space(3))) void lds_void;
+
+// size bytes per lane from buffer r at voffset + soffset into LDS at
+// lds + size * lane (lds wave-uniform).
+template <int SIZE>  // 16 or 4
+__device__ __forceinline__ void buf_to_lds(__amdgpu_buffer_rsrc_t r, void *lds, int voffset, int soffset) {
+    if constexpr (SIZE == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 16, voffset, soffset, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 4, voffset, soffset, 0, 0);
+}
+
 }  // namespace chip

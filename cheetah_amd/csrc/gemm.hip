@@ -470,16 +470,6 @@ constexpr int vm_wait_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 <<
 template <int FMT>
 constexpr int w_row_bytes() { return FMT == FMT_BF16 ? 64 : FMT == FMT_Q8 ? 32 : 16; }
 
-typedef __attribute__((address_space(3))) void lds_void;
-
-// size bytes per lane from buffer r at voffset + soffset into LDS at
-// lds + size * lane (lds wave-uniform).
-template <int SIZE>  // 16 or 4
-__device__ __forceinline__ void buf_to_lds(__amdgpu_buffer_rsrc_t r, void *lds, int voffset, int soffset) {
-    if constexpr (SIZE == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 16, voffset, soffset, 0, 0);
-    else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 4, voffset, soffset, 0, 0);
-}
-
 // ---------------------------------------------------------------------------
 // Ring GEMM, every weight format (x pre-split, K % 32 == 0): WM x WN waves of
 // 32 MT tokens x 64 weight rows (DUAL: 32 gate and the matching 32 up rows).
