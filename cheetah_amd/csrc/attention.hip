@@ -756,14 +756,13 @@ __device__ __forceinline__ void store_prefill_rows(const AttnArgs &a, const f32x
     constexpr int UT = HD / 32;
     if (S == 1) {
         const float inv = 1.0f / l;
-        float *o = a.out + ob;
 #pragma unroll
         for (int u = 0; u < UT; ++u)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const f32x4 v = f32x4{oacc[u][4 * q] * inv, oacc[u][4 * q + 1] * inv, oacc[u][4 * q + 2] * inv,
                                       oacc[u][4 * q + 3] * inv};
-                *(f32x4 *)(o + 32 * u + 8 * q + 4 * half) = v;
+                if (a.out) *(f32x4 *)(a.out + ob + 32 * u + 8 * q + 4 * half) = v;
                 if (a.out_hi) store_halves4(a.out_hi, a.out_lo, ob + 32 * u + 8 * q + 4 * half, v);
             }
     } else {
@@ -1298,7 +1297,7 @@ __global__ __launch_bounds__(kThreads) void attn_merge2_kernel(const float *part
     for (int k = 0; k < DPL; ++k) {
         const size_t i = (size_t)item * HD + lane + 64 * k;
         const float v = o[k] * inv;
-        out[i] = v;
+        if (out) out[i] = v;
         if (out_hi) {
             const __bf16 hb = (__bf16)v;
             out_hi[i] = __builtin_bit_cast(uint16_t, hb);
@@ -1460,7 +1459,8 @@ bool attention_prefill_on_mfma(const KvGeom &g, int q_heads) {
 
 int launch_attention(const AttnJob &j, hipStream_t s) {
     if (j.rows == 0) return 0;
-    if ((!j.q && !j.qkv) || !j.out || !j.k || !j.v || !j.g.page_table || (!j.prefill && j.splits > 1 && !j.part))
+    const bool halves_only = j.prefill && j.out_hi && attention_prefill_on_mfma(j.g, j.q_heads);
+    if ((!j.q && !j.qkv) || (!j.out && !halves_only) || !j.k || !j.v || !j.g.page_table || (!j.prefill && j.splits > 1 && !j.part))
         return fail("HIP backend: attention is missing a buffer.");
     if (j.g.kv_heads <= 0 || j.q_heads <= 0 || j.q_heads % j.g.kv_heads)
         return fail("HIP backend: q_heads must be a multiple of kv_heads.");

@@ -242,7 +242,7 @@ __device__ __forceinline__ void epilogue(const GArgs &a, int m, int n, float v, 
         if (a.sc2) u = u * a.sc2[n];
         // silu_multiply, ops.rs:743-747: g * (u / (1 + exp(-g))).
         const float g = v * (u / (1.0f + expf(-v)));
-        a.y[o] = g;
+        if (a.y) a.y[o] = g;
         if (a.yh) {
             const __bf16 hb = (__bf16)g;
             a.yh[o] = __builtin_bit_cast(uint16_t, hb);
@@ -290,7 +290,7 @@ __device__ __forceinline__ void epilogue_tile(const GArgs &a, const f32x16 (&tot
                     if (a.sc2) u = u * sc2n;
                     // silu_multiply, ops.rs:743-747: g * (u / (1 + exp(-g))).
                     const float g = v * (u / (1.0f + expf(-v)));
-                    a.y[o] = g;
+                    if (a.y) a.y[o] = g;
                     if (a.yh) {
                         const __bf16 hb = (__bf16)g;
                         a.yh[o] = __builtin_bit_cast(uint16_t, hb);
@@ -581,12 +581,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_ring_kernel(GArgs a, int
         const int n = min(n0 + (w_up(i) ? r - BNR / 2 : r), a.N - 1);
         woff[i] = n * (int)a.stride + byte;
     }
-    // Copy d (0 .. D - 1) of this wave's copies of stage st into ring slot
-    // st % NS (stages past the range re-read the last one into a free slot,
-    // so every wave issues the same count).
-    auto issue1 = [&](int st, int d) {
+    // Stage st sits in ring slot st % NS; the loop keeps the byte offsets of
+    // the slots it uses and advances them (no division on the scalar unit).
+    auto next_slot = [&](int off) { return off == (NS - 1) * SLOT ? 0 : off + SLOT; };
+    // Copy d (0 .. D - 1) of this wave's copies of stage st into the slot at
+    // `off` (stages past the range re-read the last one into a free slot, so
+    // every wave issues the same count).
+    auto issue1 = [&](int st, int off, int d) {
         const int k0 = kbeg + min(st, nst - 1) * BK;
-        uint8_t *slot = ring + (st % NS) * SLOT;
+        uint8_t *slot = ring + off;
         constexpr int XI = NIX / WV;
         if (d < 2 * XI) {
             const int i = d >> 1, q = wave + WV * i;
@@ -607,9 +610,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_ring_kernel(GArgs a, int
     // otherwise wait for every copy before them. The copies they need were
     // awaited explicitly, and each read waits for its data inside its own asm
     // statement, so no use of the result can be scheduled ahead of the wait.
-    auto convert = [&](int st) {
+    auto convert = [&](int st, int off) {
         constexpr int TPR = 32 / CPT, RB = FMT == FMT_Q8 ? CPT : CPT / 2;
-        const uint8_t *slot = ring + (st % NS) * SLOT + 2 * XB;
+        const uint8_t *slot = ring + off + 2 * XB;
         const int row = threadIdx.x / TPR, h = threadIdx.x % TPR;
         const uint32_t addr = (uint32_t)(uintptr_t)(slot + row * WRB + RB * h);
         u32x4 rv;
@@ -658,10 +661,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_ring_kernel(GArgs a, int
     struct Frags {
         bf16x8 ah[MT], al[MT], bw[2];
     };
-    // Fragment read d (0 .. NR - 1) of k-step k of stage st.
+    // Fragment read d (0 .. NR - 1) of k-step k of stage st in the slot at off.
     constexpr int NR = 2 + 2 * MT;
-    auto read1 = [&](int st, int k, int d, Frags &f) {
-        const uint8_t *xs = ring + (st % NS) * SLOT;
+    auto read1 = [&](int st, int off, int k, int d, Frags &f) {
+        const uint8_t *xs = ring + off;
         const uint8_t *wt = CONV ? wcv + (st & 1) * WCB : xs + 2 * XB;
         const int c = 2 * k + (lane >> 5);
         if (d < 2) {
@@ -681,16 +684,16 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_ring_kernel(GArgs a, int
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(t < 2 * MT ? f.ah[i] : f.al[i], f.bw[j], acc[i][j], 0, 0, 0);
     };
     // One k-step: the MFMAs of f with the reads of the next k-step into g and
-    // copies d0 .. d1 - 1 of stage sti between them.
+    // copies d0 .. d1 - 1 of stage sti into the slot at wr between them.
     constexpr int RPM = 2;  // fragment reads per MFMA, until all are issued
-    auto kstep = [&](const Frags &f, Frags &g, int st, int k, int sti, int d0, int d1) {
+    auto kstep = [&](const Frags &f, Frags &g, int st, int rd, int k, int sti, int wr, int d0, int d1) {
 #pragma unroll
         for (int t = 0; t < NM; ++t) {
             mma1(f, t);
 #pragma unroll
-            for (int d = RPM * t; d < min(RPM * t + RPM, NR); ++d) read1(st, k, d, g);
+            for (int d = RPM * t; d < min(RPM * t + RPM, NR); ++d) read1(st, rd, k, d, g);
 #pragma unroll
-            for (int d = d0 + t * (d1 - d0) / NM; d < d0 + (t + 1) * (d1 - d0) / NM; ++d) issue1(sti, d);
+            for (int d = d0 + t * (d1 - d0) / NM; d < d0 + (t + 1) * (d1 - d0) / NM; ++d) issue1(sti, wr, d);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -703,19 +706,22 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_ring_kernel(GArgs a, int
 #pragma unroll
     for (int st = 0; st < NS - 1; ++st)
 #pragma unroll
-        for (int d = 0; d < (st == NS - 2 ? DH : D); ++d) issue1(st, d);
+        for (int d = 0; d < (st == NS - 2 ? DH : D); ++d) issue1(st, st * SLOT, d);
     __builtin_amdgcn_s_waitcnt(vm_wait_imm(D * (CONV ? NS - 4 : NS - 3) + DH));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if constexpr (CONV) {
-        convert(0);
-        convert(1);
+        convert(0, 0);
+        convert(1, SLOT);
         __builtin_amdgcn_s_waitcnt(vm_wait_imm(63) & ~(0xF << 8));  // lgkmcnt(0)
         __builtin_amdgcn_s_barrier();
     }
     Frags f0, f1;
 #pragma unroll
-    for (int d = 0; d < NR; ++d) read1(0, 0, d, f0);
+    for (int d = 0; d < NR; ++d) read1(0, 0, 0, d, f0);
+    // Slots of stage st, of the one before it (the next copies' target) and of
+    // the copies begun in the previous iteration.
+    int rd = 0, wr = (NS - 1) * SLOT, wr_prev = (NS - 2) * SLOT;
     const int cs = a.chunk / BK;  // stages per accumulation chunk
     // Stages [s0, s1), whole chunks, folded into tot.
     auto run = [&](int s0, int s1) {
@@ -726,13 +732,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_ring_kernel(GArgs a, int
 #pragma unroll
                 for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
             for (int st = c0; st < c1; ++st) {
-                kstep(f0, f1, st, 1, st + NS - 2, DH, D);
+                kstep(f0, f1, st, rd, 1, st + NS - 2, wr_prev, DH, D);
                 __builtin_amdgcn_s_waitcnt(vm_wait_imm(D * (CONV ? NS - 4 : NS - 3)));
                 __builtin_amdgcn_s_waitcnt(vm_wait_imm(63) & ~(0xF << 8));  // lgkmcnt(0)
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
-                kstep(f1, f0, st + 1, 0, st + NS - 1, 0, DH);  // past the last stage: stale bytes, unused
-                if constexpr (CONV) convert(st + 2);
+                const int nx = next_slot(rd);
+                kstep(f1, f0, st + 1, nx, 0, st + NS - 1, wr, 0, DH);  // past the last stage: stale bytes, unused
+                if constexpr (CONV) convert(st + 2, next_slot(nx));
+                wr_prev = wr;
+                wr = rd;
+                rd = nx;
             }
             constexpr float cs16 = FMT == FMT_Q4 ? 0.0625f : 1.0f;
 #pragma unroll
@@ -1036,16 +1046,23 @@ size_t gemm_split_workspace_floats(int fmt, size_t N, size_t K, size_t m_max, bo
     return need;
 }
 
+bool gemm_takes_halves(size_t K) { return K % 8 == 0; }
+
 int launch_gemm(const GemmJob &job, hipStream_t s) {
     const WMat &w = job.w;
     if (job.n == 0) return 0;
-    if (!w.base || !job.x || w.rows == 0 || w.cols == 0) return fail("HIP backend: gemm needs a weight and an input.");
+    // Pre-split halves are used when every 8-element chunk is 16-byte aligned;
+    // x itself is then not read.
+    const bool pre = job.xh && job.xl && gemm_takes_halves(w.cols) && ((uintptr_t)job.xh % 16) == 0 &&
+                     ((uintptr_t)job.xl % 16) == 0;
+    if (!w.base || (!job.x && !pre) || w.rows == 0 || w.cols == 0)
+        return fail("HIP backend: gemm needs a weight and an input.");
     if (w.rows > (size_t)INT32_MAX || w.cols > (size_t)INT32_MAX || job.n > 65535u * 64u)
         return fail("HIP backend: gemm shape too large.");
     const bool dual = job.epi == EPI_SWIGLU;
     if (dual && (!job.w2.base || job.w2.fmt != w.fmt || job.w2.rows != w.rows || job.w2.cols != w.cols))
         return fail("HIP backend: SwiGLU gemm needs gate and up matrices of one shape and format.");
-    if (job.epi == EPI_RESIDUAL ? !job.residual : !job.y) return fail("HIP backend: gemm has no output.");
+    if (job.epi == EPI_RESIDUAL ? !job.residual : !job.y && !(dual && job.yh)) return fail("HIP backend: gemm has no output.");
     GArgs a{};
     a.w = w.payload();
     a.sc = w.scales();
@@ -1069,8 +1086,6 @@ int launch_gemm(const GemmJob &job, hipStream_t s) {
     a.nchunks = (a.K + a.chunk - 1) / a.chunk;
     a.ws = job.ws;
     a.vec_x = (a.K % 4) == 0 && ((uintptr_t)job.x % 16) == 0;
-    // Pre-split halves are used when every 8-element chunk is 16-byte aligned.
-    const bool pre = job.xh && job.xl && a.K % 8 == 0 && ((uintptr_t)job.xh % 16) == 0 && ((uintptr_t)job.xl % 16) == 0;
     a.xh = pre ? job.xh : nullptr;
     a.xl = pre ? job.xl : nullptr;
     const uintptr_t p1 = (uintptr_t)a.w, p2 = dual ? (uintptr_t)a.w2 : p1;

@@ -59,9 +59,11 @@ struct GemmJob {
     // Optional x pre-split by launch_split_bf16 ([n][cols] each): the GEMM
     // then stages BF16 halves instead of splitting x once per weight tile
     // (the same bits).
+    // x may be null where gemm_takes_halves(cols).
     const uint16_t *xh = nullptr, *xl = nullptr;
     // EPI_SWIGLU only, optional: the output also as BF16 halves ([n][rows]
-    // each, the bits launch_split_bf16 would give), for the next GEMM.
+    // each, the bits launch_split_bf16 would give), for the next GEMM; y may
+    // then be null.
     uint16_t *yh = nullptr, *yl = nullptr;
     // EPI_RESIDUAL / EPI_STORE, optional: when the GEMM splits K, leave the
     // stored sums in ws ([*deferred][n][rows]: every chunk's, or the two
@@ -71,6 +73,8 @@ struct GemmJob {
     int *deferred = nullptr;
 };
 int launch_gemm(const GemmJob &job, hipStream_t stream);
+// Whether a GEMM over K columns given xh / xl reads them and not x.
+bool gemm_takes_halves(size_t K);
 int launch_split_bf16(const float *x, size_t n, uint16_t *xh, uint16_t *xl, hipStream_t s);
 int gemm_chunk_depth(int K);
 // Split-K scratch a GEMM of M tokens uses; with less it runs another split
@@ -93,7 +97,8 @@ int launch_embed(const uint16_t *table, size_t hidden, const uint32_t *tokens, s
                  hipStream_t s);
 // out[i][:] = rmsnorm(x[i][:]) * gain (rows of width n)
 // Row-wise RMSNorm; with xh / xl also the normed rows as BF16 halves (the
-// bits launch_split_bf16 would give), the MFMA GEMM's input.
+// bits launch_split_bf16 would give), the MFMA GEMM's input; out may then be
+// null.
 int launch_rmsnorm_rows(const float *x, const uint16_t *gain, float eps, size_t rows, size_t n, float *out,
                         hipStream_t s, uint16_t *xh = nullptr, uint16_t *xl = nullptr);
 // A deferred residual GEMM's reduction fused with the next RMSNorm: per row
@@ -101,7 +106,7 @@ int launch_rmsnorm_rows(const float *x, const uint16_t *gain, float eps, size_t 
 // GEMM folds them (the first ceil(n / 2) in order, the rest in order, the
 // two added), times
 // sc[i], plus bias[i] (each optional), hidden[m][i] += v; then, with a gain,
-// the row RMSNorm of hidden into out (and BF16 halves when xh / xl are set).
+// the row RMSNorm of hidden into out and / or BF16 halves (xh / xl).
 // The same operations as the GEMM's split-K reduction then
 // launch_rmsnorm_rows.
 int launch_residual_rmsnorm_rows(const float *ws, int nchunks, const float *sc, const float *bias, float *hidden,
@@ -186,7 +191,8 @@ struct AttnJob {
     int rotary_dim = 0;
     // Chunked prefill on the matrix cores (attention_prefill_on_mfma) also
     // writes out's BF16 halves here when set: hi = bf16(v), lo = bf16(v - hi),
-    // the bits launch_split_bf16 would write. Other paths ignore them.
+    // the bits launch_split_bf16 would write; out may then be null. Other
+    // paths ignore them.
     uint16_t *out_hi = nullptr, *out_lo = nullptr;
 };
 int launch_attention(const AttnJob &job, hipStream_t s);

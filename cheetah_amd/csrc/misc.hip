@@ -31,7 +31,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_rows_kernel(const float *x, 
                                                                 float *out, uint16_t *xh, uint16_t *xl) {
     __shared__ float red[kThreads / 64];
     const float *src = x + (size_t)blockIdx.x * n;
-    float *dst = out + (size_t)blockIdx.x * n;
+    float *dst = out ? out + (size_t)blockIdx.x * n : nullptr;
     // Eight of the thread's elements loaded at a time; squares summed in
     // element order.
     float ss = 0.f;
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_rows_kernel(const float *x, 
     const float inv = 1.0f / sqrtf(total / (float)n + eps);
     for (int i = threadIdx.x; i < n; i += kThreads) {
         const float v = src[i] * (inv * bf16_f32(gain[i]));
-        dst[i] = v;
+        if (dst) dst[i] = v;
         if (xh) {
             const size_t o = (size_t)blockIdx.x * n + i;
             const __bf16 hb = (__bf16)v;
@@ -130,10 +130,10 @@ __global__ __launch_bounds__(kThreads) void residual_rmsnorm_rows_kernel(const f
     __syncthreads();
     const float total = red[0] + red[1] + red[2] + red[3];
     const float inv = 1.0f / sqrtf(total / (float)n + eps);
-    float *dst = out + (size_t)m * n;
+    float *dst = out ? out + (size_t)m * n : nullptr;
     for (int i = threadIdx.x; i < n; i += kThreads) {
         const float v = h[i] * (inv * bf16_f32(gain[i]));
-        dst[i] = v;
+        if (dst) dst[i] = v;
         if (xh) {
             const size_t o = (size_t)m * n + i;
             const __bf16 hb = (__bf16)v;
@@ -198,13 +198,13 @@ __global__ __launch_bounds__(kThreads) void residual_rmsnorm_rows_reg_kernel(con
     __syncthreads();
     const float total = red[0] + red[1] + red[2] + red[3];
     const float inv = 1.0f / sqrtf(total / (float)n + eps);
-    float *dst = out + (size_t)m * n;
+    float *dst = out ? out + (size_t)m * n : nullptr;
 #pragma unroll
     for (int k = 0; k < EPT; ++k) {
         const int i = (int)threadIdx.x + kThreads * k;
         if (i < n) {
             const float v = r[k] * (inv * gv[k]);
-            dst[i] = v;
+            if (dst) dst[i] = v;
             if (xh) {
                 const size_t o = (size_t)m * n + i;
                 const __bf16 hb = (__bf16)v;
@@ -385,7 +385,7 @@ int launch_residual_rmsnorm_rows(const float *ws, int nchunks, const float *sc, 
                                  size_t rows, size_t n, const uint16_t *gain, float eps, float *out, hipStream_t s,
                                  uint16_t *xh, uint16_t *xl) {
     if (rows == 0) return 0;
-    if (!ws || nchunks <= 0 || !hidden || (gain && !out)) return fail("HIP backend: residual norm is missing a buffer.");
+    if (!ws || nchunks <= 0 || !hidden || (gain && !out && !xh)) return fail("HIP backend: residual norm is missing a buffer.");
     if (!xh != !xl) return fail("HIP backend: rmsnorm needs both BF16 halves or neither.");
     if (rows > (size_t)INT32_MAX || n > (size_t)INT32_MAX) return fail("HIP backend: residual norm shape too large.");
     // A row of 1,025 to 4,096 with at most four stored sums (a GEMM's two halves) in registers: one load round

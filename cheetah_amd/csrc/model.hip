@@ -995,6 +995,11 @@ int enqueue_chunk(cheetah_hip_model *m, const uint32_t *tokens_dev, size_t rows,
     // reduction then runs fused with the RMSNorm that reads its output.
     int down_chunks = 0;
     const float *down_sc = nullptr;
+    // The GEMMs read BF16 halves: f32 copies of their inputs are written only
+    // where a width rules the halves out.
+    float *normed = gemm_takes_halves(H) ? nullptr : m->normed;
+    float *attn = gemm_takes_halves(sh.q_dim()) ? nullptr : m->attn;
+    float *act = gemm_takes_halves(c.intermediate_size) ? nullptr : m->act;
     for (uint32_t l = 0; l < c.num_layers; ++l) {
         const Layer *Lp = nullptr;
         CHIP_TRY(layer_begin(m, l, s, &Lp));
@@ -1002,12 +1007,12 @@ int enqueue_chunk(cheetah_hip_model *m, const uint32_t *tokens_dev, size_t rows,
         // The normed rows come with their BF16 halves (the GEMM's input).
         if (down_chunks)
             CHIP_TRY(launch_residual_rmsnorm_rows(m->gemm_ws, down_chunks, down_sc, nullptr, m->hidden, rows, H, L.ln1,
-                                                  c.rms_eps, m->normed, s, m->xh, m->xl));
+                                                  c.rms_eps, normed, s, m->xh, m->xl));
         else
-            CHIP_TRY(launch_rmsnorm_rows(m->hidden, L.ln1, c.rms_eps, rows, H, m->normed, s, m->xh, m->xl));
+            CHIP_TRY(launch_rmsnorm_rows(m->hidden, L.ln1, c.rms_eps, rows, H, normed, s, m->xh, m->xl));
         GemmJob qkv;
         qkv.w = L.qkv;
-        qkv.x = m->normed;
+        qkv.x = normed;
         qkv.n = rows;
         qkv.bias = L.qkv_bias;
         qkv.y = m->qkv;
@@ -1026,7 +1031,7 @@ int enqueue_chunk(cheetah_hip_model *m, const uint32_t *tokens_dev, size_t rows,
         AttnJob aj;
         aj.q = m->qrot;
         aj.q_stride = sh.q_dim();
-        aj.out = m->attn;
+        aj.out = attn;
         aj.k = L.kv.k;
         aj.v = L.kv.v;
         aj.g = geom(m);
@@ -1046,7 +1051,7 @@ int enqueue_chunk(cheetah_hip_model *m, const uint32_t *tokens_dev, size_t rows,
         CHIP_TRY(launch_attention(aj, s));
         GemmJob o;
         o.w = L.o;
-        o.x = m->attn;
+        o.x = attn;
         o.n = rows;
         o.bias = L.o_bias;
         o.residual = m->hidden;
@@ -1060,15 +1065,15 @@ int enqueue_chunk(cheetah_hip_model *m, const uint32_t *tokens_dev, size_t rows,
         CHIP_TRY(launch_gemm(o, s));
         if (o_chunks)
             CHIP_TRY(launch_residual_rmsnorm_rows(m->gemm_ws, o_chunks, L.o.scales(), L.o_bias, m->hidden, rows, H,
-                                                  L.ln2, c.rms_eps, m->normed, s, m->xh, m->xl));
+                                                  L.ln2, c.rms_eps, normed, s, m->xh, m->xl));
         else
-            CHIP_TRY(launch_rmsnorm_rows(m->hidden, L.ln2, c.rms_eps, rows, H, m->normed, s, m->xh, m->xl));
+            CHIP_TRY(launch_rmsnorm_rows(m->hidden, L.ln2, c.rms_eps, rows, H, normed, s, m->xh, m->xl));
         GemmJob gu;
         gu.w = L.gate;
         gu.w2 = L.up;
-        gu.x = m->normed;
+        gu.x = normed;
         gu.n = rows;
-        gu.y = m->act;
+        gu.y = act;
         gu.epi = EPI_SWIGLU;
         gu.ws = m->gemm_ws;
         gu.ws_floats = m->gemm_ws_floats;
@@ -1079,7 +1084,7 @@ int enqueue_chunk(cheetah_hip_model *m, const uint32_t *tokens_dev, size_t rows,
         CHIP_TRY(launch_gemm(gu, s));
         GemmJob dn;
         dn.w = L.down;
-        dn.x = m->act;
+        dn.x = act;
         dn.n = rows;
         dn.residual = m->hidden;
         dn.epi = EPI_RESIDUAL;
