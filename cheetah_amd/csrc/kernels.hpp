@@ -221,4 +221,13 @@ int launch_argmax(const float *logits, size_t n, uint32_t *out_token, int32_t *s
                   size_t hist_cap, void *scratch, hipStream_t s);
 size_t argmax_scratch_bytes();
 
+// step[0] = token, step[1] = pos, in stream order.
+int launch_set_step(int32_t *step, int32_t token, int32_t pos, hipStream_t s);
+// A forward's results into pinned host memory (device addresses of it): n
+// logits when `logits` is set, words[0] = *token, words[1] = *abort_flag (0
+// when null). One kernel in stream order takes the place of a copy per result,
+// each of which cost the copy engine's round trip.
+int launch_export(const float *logits, size_t n, float *logits_out, const uint32_t *token, const int32_t *abort_flag,
+                  int32_t *words, hipStream_t s);
+
 }  // namespace chip

@@ -360,7 +360,51 @@ __global__ __launch_bounds__(kThreads) void argmax_final_kernel(const int *pkey,
     }
 }
 
+// step[0] = token, step[1] = position (both in the launch's arguments: no
+// host buffer to copy from, nothing to wait for).
+__global__ void set_step_kernel(int32_t *step, int32_t token, int32_t pos) {
+    step[0] = token;
+    step[1] = pos;
+}
+
+// A forward's results into pinned host memory: the logits (when asked for)
+// and words[0] = the sampled token, words[1] = the abort flag (0 without one).
+__global__ __launch_bounds__(kThreads) void export_kernel(const float *logits, int n, float *logits_out,
+                                                          const uint32_t *token, const int32_t *abort_flag,
+                                                          int32_t *words) {
+    const int i = 4 * (int)(blockIdx.x * kThreads + threadIdx.x);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        words[0] = (int32_t)*token;
+        words[1] = abort_flag ? *abort_flag : 0;
+    }
+    if (!logits) return;
+    if (i + 4 <= n) {
+        *(f32x4 *)(logits_out + i) = *(const f32x4 *)(logits + i);
+    } else {
+        for (int k = i; k < n; ++k) logits_out[k] = logits[k];
+    }
+}
+
 }  // namespace
+
+int launch_set_step(int32_t *step, int32_t token, int32_t pos, hipStream_t s) {
+    if (!step) return fail("HIP backend: no step words.");
+    hipLaunchKernelGGL(set_step_kernel, dim3(1), dim3(1), 0, s, step, token, pos);
+    CHIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+int launch_export(const float *logits, size_t n, float *logits_out, const uint32_t *token, const int32_t *abort_flag,
+                  int32_t *words, hipStream_t s) {
+    if (!token || !words || (logits && (!logits_out || n == 0 || n > (size_t)INT32_MAX)))
+        return fail("HIP backend: export is missing a buffer.");
+    if (((uintptr_t)logits | (uintptr_t)logits_out) % 16) return fail("HIP backend: export needs 16-byte aligned logits.");
+    const unsigned blocks = logits ? (unsigned)((n + 4 * kThreads - 1) / (4 * kThreads)) : 1u;
+    hipLaunchKernelGGL(export_kernel, dim3(blocks), dim3(kThreads), 0, s, logits, (int)n, logits_out, token, abort_flag,
+                       words);
+    CHIP_CHECK(hipGetLastError());
+    return 0;
+}
 
 int launch_embed(const uint16_t *table, size_t hidden, const uint32_t *tokens, size_t rows, float *out,
                  hipStream_t s) {

@@ -204,9 +204,11 @@ struct cheetah_hip_model {
     uint32_t *tokens_dev = nullptr, *next_dev = nullptr, *hist_dev = nullptr;
     int32_t *step_dev = nullptr;  // [0] = token, [1] = position
     void *argmax_scratch = nullptr;
-    int32_t *step_host = nullptr;    // pinned
+    int32_t *words_host = nullptr;   // pinned: [0] = sampled token, [1] = abort flag (launch_export)
+    int32_t *words_out = nullptr;    // its device address
     uint32_t *tokens_host = nullptr;  // pinned staging for chunk tokens
     float *logits_host = nullptr;     // pinned
+    float *logits_out = nullptr;      // its device address
     // Decode graphs, one per attention split count (the grid of a captured
     // launch is fixed; the split count follows the context length).
     std::vector<hipGraphExec_t> graphs = std::vector<hipGraphExec_t>(attention_max_splits() + 1, nullptr);
@@ -220,7 +222,6 @@ struct cheetah_hip_model {
     size_t tagged_words = 0;
     int32_t *abort_dev = nullptr;
     unsigned next_tag = 1;          // tag of the next launch's first phase
-    int32_t *abort_host = nullptr;  // pinned
     unsigned epoch = 0;             // the weight epoch the graphs and layer table were built for
     // Host-tier feed: layer l's streamed matrices are copied from pinned
     // host memory into slot l % 2 on feed_stream, one streamed layer ahead
@@ -247,10 +248,9 @@ struct cheetah_hip_model {
         for (hipGraphExec_t g : graphs)
             if (g) (void)hipGraphExecDestroy(g);
         if (stream) (void)hipStreamDestroy(stream);
-        if (step_host) (void)hipHostFree(step_host);
+        if (words_host) (void)hipHostFree(words_host);
         if (tokens_host) (void)hipHostFree(tokens_host);
         if (logits_host) (void)hipHostFree(logits_host);
-        if (abort_host) (void)hipHostFree(abort_host);
         for (int p : pages) sh->page_unref(p);
     }
 };
@@ -510,7 +510,6 @@ int init_fused(cheetah_hip_model *m) {
     CHIP_TRY(m->mem.alloc(&m->abort_dev, 1));
     CHIP_CHECK(hipMemset(m->abort_dev, 0, sizeof(int32_t)));
     m->next_tag = 1;
-    CHIP_CHECK(hipHostMalloc((void **)&m->abort_host, sizeof(int32_t), hipHostMallocDefault));
     return 0;
 }
 
@@ -562,9 +561,10 @@ int ensure_down_cols(cheetah_hip_model *m) {
 
 // Runs `steps` decode steps in one persistent launch from the token and
 // position (`offset`, also in step_dev); leaves the last step's logits in
-// m->logits, its argmax in next_dev and every sampled id in hist_dev. Waits
+// m->logits (with want_logits also in logits_host), its argmax in step_dev and
+// words_host[0], and every sampled id in hist_dev. Waits
 // for the launch.
-int run_fused(cheetah_hip_model *m, size_t offset, size_t steps) {
+int run_fused(cheetah_hip_model *m, size_t offset, size_t steps, bool want_logits = false) {
     Shared &sh = *m->sh;
     const auto &c = sh.cfg;
     CHIP_TRY(ensure_down_cols(m));
@@ -635,10 +635,10 @@ int run_fused(cheetah_hip_model *m, size_t offset, size_t steps) {
         }
     }
     m->next_tag += (unsigned)steps * per_step;
-    CHIP_CHECK(hipMemcpyAsync(m->next_dev, m->step_dev, sizeof(uint32_t), hipMemcpyDeviceToDevice, m->stream));
-    CHIP_CHECK(hipMemcpyAsync(m->abort_host, m->abort_dev, sizeof(int32_t), hipMemcpyDeviceToHost, m->stream));
+    CHIP_TRY(launch_export(want_logits ? m->logits : nullptr, c.vocab_size, m->logits_out,
+                           (const uint32_t *)m->step_dev, m->abort_dev, m->words_out, m->stream));
     CHIP_CHECK(hipStreamSynchronize(m->stream));
-    if (*m->abort_host) {
+    if (m->words_host[1]) {
         // A poll timed out: the steps are incomplete. Reset the hand-off
         // words so the next launch starts clean.
         CHIP_CHECK(hipMemset(m->tagged, 0, m->tagged_words * sizeof(uint64_t)));
@@ -698,9 +698,11 @@ int init_instance(cheetah_hip_model *m) {
     CHIP_TRY(m->mem.alloc(&scratch, argmax_scratch_bytes()));
     m->argmax_scratch = scratch;
     CHIP_TRY(m->mem.alloc(&m->page_dev, (size_t)sh.num_pages));
-    CHIP_CHECK(hipHostMalloc((void **)&m->step_host, 2 * sizeof(int32_t), hipHostMallocDefault));
+    CHIP_CHECK(hipHostMalloc((void **)&m->words_host, 2 * sizeof(int32_t), hipHostMallocDefault));
+    CHIP_CHECK(hipHostGetDevicePointer((void **)&m->words_out, m->words_host, 0));
     CHIP_CHECK(hipHostMalloc((void **)&m->tokens_host, sh.kv_capacity * sizeof(uint32_t), hipHostMallocDefault));
     CHIP_CHECK(hipHostMalloc((void **)&m->logits_host, (size_t)c.vocab_size * sizeof(float), hipHostMallocDefault));
+    CHIP_CHECK(hipHostGetDevicePointer((void **)&m->logits_out, m->logits_host, 0));
     m->page_host.assign(sh.num_pages, 0);
     return init_fused(m);
 }
@@ -975,14 +977,6 @@ int launch_decode(cheetah_hip_model *m, size_t pos) {
     return 0;
 }
 
-int write_step(cheetah_hip_model *m, uint32_t token, size_t pos) {
-    CHIP_CHECK(hipStreamSynchronize(m->stream));  // step_host may still be in flight
-    m->step_host[0] = (int32_t)token;
-    m->step_host[1] = (int32_t)pos;
-    CHIP_CHECK(hipMemcpyAsync(m->step_dev, m->step_host, 2 * sizeof(int32_t), hipMemcpyHostToDevice, m->stream));
-    return 0;
-}
-
 // One prefill chunk of `rows` tokens at absolute position `pos`.
 // tokens_dev holds the chunk's ids (already on the device).
 int enqueue_chunk(cheetah_hip_model *m, const uint32_t *tokens_dev, size_t rows, size_t pos, bool last_chunk) {
@@ -1148,9 +1142,10 @@ int validate_decode(const cheetah_hip_model *m, uint32_t token, size_t offset, s
     return 0;
 }
 
-// Runs the forward; leaves the final logits in m->logits (and, for decode,
-// the argmax in m->next_dev).
-int run_forward(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t offset, size_t chunk_rows) {
+// Runs the forward and waits for it; leaves the argmax in words_host[0] and,
+// with want_logits, the final logits in logits_host.
+int run_forward(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t offset, size_t chunk_rows,
+                bool want_logits) {
     CHIP_TRY(check_model(m));
     CHIP_TRY(validate(m, tokens, n, offset));
     CHIP_TRY(refresh_weights(m));
@@ -1158,9 +1153,13 @@ int run_forward(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t o
     chunk_rows = std::min(chunk_rows, m->sh->max_chunk);
     CHIP_TRY(reserve_positions(m, n));
     if (n == 1) {
-        CHIP_TRY(write_step(m, tokens[0], offset));
-        if (fused_fits(m, offset, 1)) CHIP_TRY(run_fused(m, offset, 1));
-        else CHIP_TRY(launch_decode(m, offset));
+        CHIP_TRY(launch_set_step(m->step_dev, (int32_t)tokens[0], (int32_t)offset, m->stream));
+        if (fused_fits(m, offset, 1)) {
+            CHIP_TRY(run_fused(m, offset, 1, want_logits));
+            m->len = offset + 1;
+            return 0;
+        }
+        CHIP_TRY(launch_decode(m, offset));
     } else {
         CHIP_CHECK(hipStreamSynchronize(m->stream));  // tokens_host reuse
         std::memcpy(m->tokens_host, tokens, n * sizeof(uint32_t));
@@ -1173,6 +1172,9 @@ int run_forward(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t o
         CHIP_TRY(launch_argmax(m->logits, C(m).vocab_size, m->next_dev, nullptr, nullptr, 0, m->argmax_scratch,
                                m->stream));
     }
+    CHIP_TRY(launch_export(want_logits ? m->logits : nullptr, C(m).vocab_size, m->logits_out, m->next_dev, nullptr,
+                           m->words_out, m->stream));
+    CHIP_CHECK(hipStreamSynchronize(m->stream));
     m->len = offset + n;
     return 0;
 }
@@ -1203,14 +1205,6 @@ bool parse_layer_unit(const Shared &sh, const char *id, uint32_t *layer, int *ma
             return true;
         }
     return false;
-}
-
-int read_logits(cheetah_hip_model *m, float *logits_out) {
-    const size_t V = C(m).vocab_size;
-    CHIP_CHECK(hipMemcpyAsync(m->logits_host, m->logits, V * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-    CHIP_CHECK(hipStreamSynchronize(m->stream));
-    std::memcpy(logits_out, m->logits_host, V * sizeof(float));
-    return 0;
 }
 
 }  // namespace
@@ -1303,18 +1297,17 @@ int cheetah_hip_model_finalize(cheetah_hip_model *m) {
 int cheetah_hip_forward(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t offset, size_t chunk_rows,
                         float *logits_out) {
     if (!logits_out) return fail("HIP backend: null logits buffer.");
-    if (run_forward(m, tokens, n, offset, chunk_rows)) return -1;
-    return read_logits(m, logits_out);
+    if (run_forward(m, tokens, n, offset, chunk_rows, true)) return -1;
+    std::memcpy(logits_out, m->logits_host, C(m).vocab_size * sizeof(float));
+    return 0;
 }
 
 int cheetah_hip_forward_greedy(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t offset,
                                size_t chunk_rows, uint32_t *next_token, float *logits_out) {
     if (!next_token) return fail("HIP backend: null next_token pointer.");
-    if (run_forward(m, tokens, n, offset, chunk_rows)) return -1;
-    CHIP_CHECK(hipMemcpyAsync(m->step_host, m->next_dev, sizeof(uint32_t), hipMemcpyDeviceToHost, m->stream));
-    CHIP_CHECK(hipStreamSynchronize(m->stream));
-    *next_token = (uint32_t)m->step_host[0];
-    if (logits_out) CHIP_TRY(read_logits(m, logits_out));
+    if (run_forward(m, tokens, n, offset, chunk_rows, logits_out != nullptr)) return -1;
+    *next_token = (uint32_t)m->words_host[0];
+    if (logits_out) std::memcpy(logits_out, m->logits_host, C(m).vocab_size * sizeof(float));
     return 0;
 }
 
@@ -1326,7 +1319,7 @@ int cheetah_hip_decode_greedy(cheetah_hip_model *m, uint32_t token, size_t offse
     CHIP_TRY(validate_decode(m, token, offset, steps));
     CHIP_TRY(refresh_weights(m));
     CHIP_TRY(reserve_positions(m, steps));
-    CHIP_TRY(write_step(m, token, offset));
+    CHIP_TRY(launch_set_step(m->step_dev, (int32_t)token, (int32_t)offset, m->stream));
     if (fused_fits(m, offset, steps)) CHIP_TRY(run_fused(m, offset, steps));
     else
         for (size_t i = 0; i < steps; ++i) CHIP_TRY(launch_decode(m, offset + i));
@@ -1344,7 +1337,7 @@ int cheetah_hip_time_decode(cheetah_hip_model *m, uint32_t token, size_t offset,
     CHIP_TRY(validate_decode(m, token, offset, steps));
     CHIP_TRY(refresh_weights(m));
     CHIP_TRY(reserve_positions(m, steps));
-    CHIP_TRY(write_step(m, token, offset));
+    CHIP_TRY(launch_set_step(m->step_dev, (int32_t)token, (int32_t)offset, m->stream));
     hipEvent_t e0, e1;
     CHIP_CHECK(hipEventCreate(&e0));
     CHIP_CHECK(hipEventCreate(&e1));
