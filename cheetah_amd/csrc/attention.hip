@@ -1420,8 +1420,14 @@ int attention_max_splits() { return kMaxSplits; }
 // block per CU for the matrix-core kernel (BF16 K/V; measured 13 % faster
 // than two at 16K keys, where the K/V stream, not the block count, sets the
 // time) and two for the VALU kernel (f32 K/V), at most one split per
-// 64-position tile and kMaxSplits.
-int attention_decode_splits(size_t ctx, int kv_heads, size_t rows, bool kv_f32) {
+// 64-position tile and kMaxSplits. A short BF16 context takes one block per
+// KV head, which needs no merge launch: up to 256 positions at head_dim 128
+// (32 q / 8 KV heads, split -> one block: 128 keys 7.9 -> 6.2 us, 256 7.9 ->
+// 6.8, 320 7.9 -> 8.0) and 384 at 64 (14 / 2 heads: 128 6.9 -> 5.2, 384 7.1 ->
+// 6.8, 512 7.2 -> 7.5). One block of 8 or 16 waves was slower from 200 keys on
+// (512 keys, 14 / 2 heads of 64: 9.4 us).
+int attention_decode_splits(size_t ctx, int kv_heads, size_t rows, bool kv_f32, int head_dim) {
+    if (!kv_f32 && rows == 1 && ctx <= (head_dim == 64 ? 384u : 256u)) return 1;
     const size_t per_cu = kv_f32 ? 2 : 1;
     const size_t target = per_cu * (size_t)std::max(device_cus(), 1);
     const size_t per = (size_t)std::max(kv_heads, 1) * std::max<size_t>(rows, 1);

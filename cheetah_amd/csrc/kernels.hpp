@@ -202,8 +202,8 @@ bool attention_decode_fuses_rope(const KvGeom &g, int q_heads, int rotary_dim);
 size_t attention_part_floats(size_t rows, int q_heads, int splits, int head_dim);
 // Split count of a decode-style launch (one row per query position) over ctx
 // keys: one or two blocks per CU (matrix-core or VALU kernel), at most one
-// split per 64-position tile.
-int attention_decode_splits(size_t ctx, int kv_heads, size_t rows, bool kv_f32);
+// split per 64-position tile, one for a short BF16 context.
+int attention_decode_splits(size_t ctx, int kv_heads, size_t rows, bool kv_f32, int head_dim);
 int attention_max_splits();
 int attention_prefill_splits(size_t ctx, int span = kDefaultPrefillSpan);
 // A model's prefill span from its KV capacity: the largest power of two at

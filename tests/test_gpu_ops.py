@@ -203,6 +203,22 @@ def test_attention_decode_matches_oracle(hip, oracle, q_heads, kv_heads, hd, ctx
     assert np.max(np.abs(got - ref)) < 1e-4
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,hd,ctx", [(14, 2, 64, 128), (14, 2, 64, 129), (14, 2, 64, 384),
+                                                     (14, 2, 64, 385), (32, 8, 128, 97), (28, 4, 128, 256),
+                                                     (28, 4, 128, 257), (8, 1, 128, 255)])
+def test_attention_decode_around_the_one_block_limit(hip, oracle, q_heads, kv_heads, hd, ctx):
+    """Short contexts run as one block per KV head (256 keys at head_dim 128,
+    384 at 64), longer ones split and merge: the edges of both, and of the
+    rounds of four 32-key tiles. Queries and probabilities are two BF16 halves
+    (2^-17); values are N(0, 1): 2e-5 of the output's scale."""
+    rng = np.random.default_rng(ctx + hd)
+    k, v, q = _attn_case(rng, q_heads, kv_heads, hd, ctx, 1)
+    kp, vp, table = hip.paged_kv(k, v, seed=ctx)
+    got = hip.attention(q, kp, vp, table, q_heads, 1, ctx - 1)[0]
+    ref = oracle.attention(synth.bf16_to_f32(k), synth.bf16_to_f32(v), q[0], q_heads, kv_heads, hd, ctx - 1)
+    assert rel_err(got, ref) < 2e-5
+
+
 @pytest.mark.parametrize("q_heads,kv_heads,hd,offset,rows", [(14, 2, 64, 0, 37), (32, 8, 128, 100, 70),
                                                             (28, 4, 128, 4000, 9)])
 def test_attention_prefill_rows_match_oracle(hip, oracle, q_heads, kv_heads, hd, offset, rows):
