@@ -211,7 +211,9 @@ struct cheetah_hip_model {
     float *logits_out = nullptr;      // its device address
     // Decode graphs, one per attention split count (the grid of a captured
     // launch is fixed; the split count follows the context length).
-    std::vector<hipGraphExec_t> graphs = std::vector<hipGraphExec_t>(attention_max_splits() + 1, nullptr);
+    // One set without the argmax (a forward that returns only logits) and one
+    // with it.
+    std::vector<hipGraphExec_t> graphs = std::vector<hipGraphExec_t>(2 * (attention_max_splits() + 1), nullptr);
     // Persistent decode kernel state (decode_fused.hip).
     bool fused_ok = false;
     FusedLayer *fused_layers = nullptr;  // device [L]
@@ -862,8 +864,9 @@ int decode_splits(const cheetah_hip_model *m, size_t ctx) {
                                    (int)m->sh->cfg.head_dim);
 }
 
-// One decode step's kernels; token and position are read from step_dev.
-int enqueue_decode(cheetah_hip_model *m, int splits) {
+// One decode step's kernels; token and position are read from step_dev. With
+// `sample` the argmax follows and advances step_dev.
+int enqueue_decode(cheetah_hip_model *m, int splits, bool sample) {
     Shared &sh = *m->sh;
     const auto &c = sh.cfg;
     hipStream_t s = m->stream;
@@ -938,6 +941,7 @@ int enqueue_decode(cheetah_hip_model *m, int splits) {
     head.eps = c.rms_eps;
     head.y = m->logits;
     CHIP_TRY(launch_gemv(head, s));
+    if (!sample) return 0;
     CHIP_TRY(launch_argmax(m->logits, c.vocab_size, m->next_dev, m->step_dev, m->hist_dev, sh.kv_capacity + 1,
                            m->argmax_scratch, s));
     return 0;
@@ -950,17 +954,17 @@ bool graphs_enabled() {
 
 // One decode step at absolute position `pos` (the device step word must
 // already hold it): the captured graph for the step's split count.
-int launch_decode(cheetah_hip_model *m, size_t pos) {
+int launch_decode(cheetah_hip_model *m, size_t pos, bool sample) {
     const int splits = decode_splits(m, pos + 1);
     // Host-tier weights are fed by copies ordered with events on a second
     // stream: those steps run eagerly.
-    if (!graphs_enabled() || m->sh->host_mats) return enqueue_decode(m, splits);
-    if (splits < 1 || (size_t)splits >= m->graphs.size()) return fail("HIP backend: decode split count out of range.");
-    hipGraphExec_t &exec = m->graphs[splits];
+    if (!graphs_enabled() || m->sh->host_mats) return enqueue_decode(m, splits, sample);
+    if (splits < 1 || splits > attention_max_splits()) return fail("HIP backend: decode split count out of range.");
+    hipGraphExec_t &exec = m->graphs[2 * (size_t)splits + (sample ? 1 : 0)];
     if (!exec) {
         hipGraph_t g = nullptr;
         CHIP_CHECK(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-        const int rc = enqueue_decode(m, splits);
+        const int rc = enqueue_decode(m, splits, sample);
         hipError_t e = hipStreamEndCapture(m->stream, &g);
         if (rc != 0) {
             if (g) (void)hipGraphDestroy(g);
@@ -1143,10 +1147,10 @@ int validate_decode(const cheetah_hip_model *m, uint32_t token, size_t offset, s
     return 0;
 }
 
-// Runs the forward and waits for it; leaves the argmax in words_host[0] and,
-// with want_logits, the final logits in logits_host.
+// Runs the forward and waits for it; leaves, with `sample`, the argmax in
+// words_host[0] and, with want_logits, the final logits in logits_host.
 int run_forward(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t offset, size_t chunk_rows,
-                bool want_logits) {
+                bool sample, bool want_logits) {
     CHIP_TRY(check_model(m));
     CHIP_TRY(validate(m, tokens, n, offset));
     CHIP_TRY(refresh_weights(m));
@@ -1160,7 +1164,7 @@ int run_forward(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t o
             m->len = offset + 1;
             return 0;
         }
-        CHIP_TRY(launch_decode(m, offset));
+        CHIP_TRY(launch_decode(m, offset, sample));
     } else {
         CHIP_CHECK(hipStreamSynchronize(m->stream));  // tokens_host reuse
         std::memcpy(m->tokens_host, tokens, n * sizeof(uint32_t));
@@ -1170,8 +1174,9 @@ int run_forward(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t o
             const size_t rows = std::min(chunk_rows, n - start);
             CHIP_TRY(enqueue_chunk(m, m->tokens_dev + start, rows, offset + start, start + rows == n));
         }
-        CHIP_TRY(launch_argmax(m->logits, C(m).vocab_size, m->next_dev, nullptr, nullptr, 0, m->argmax_scratch,
-                               m->stream));
+        if (sample)
+            CHIP_TRY(launch_argmax(m->logits, C(m).vocab_size, m->next_dev, nullptr, nullptr, 0, m->argmax_scratch,
+                                   m->stream));
     }
     CHIP_TRY(launch_export(want_logits ? m->logits : nullptr, C(m).vocab_size, m->logits_out, m->next_dev, nullptr,
                            m->words_out, m->stream));
@@ -1298,7 +1303,7 @@ int cheetah_hip_model_finalize(cheetah_hip_model *m) {
 int cheetah_hip_forward(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t offset, size_t chunk_rows,
                         float *logits_out) {
     if (!logits_out) return fail("HIP backend: null logits buffer.");
-    if (run_forward(m, tokens, n, offset, chunk_rows, true)) return -1;
+    if (run_forward(m, tokens, n, offset, chunk_rows, false, true)) return -1;
     std::memcpy(logits_out, m->logits_host, C(m).vocab_size * sizeof(float));
     return 0;
 }
@@ -1306,7 +1311,7 @@ int cheetah_hip_forward(cheetah_hip_model *m, const uint32_t *tokens, size_t n, 
 int cheetah_hip_forward_greedy(cheetah_hip_model *m, const uint32_t *tokens, size_t n, size_t offset,
                                size_t chunk_rows, uint32_t *next_token, float *logits_out) {
     if (!next_token) return fail("HIP backend: null next_token pointer.");
-    if (run_forward(m, tokens, n, offset, chunk_rows, logits_out != nullptr)) return -1;
+    if (run_forward(m, tokens, n, offset, chunk_rows, true, logits_out != nullptr)) return -1;
     *next_token = (uint32_t)m->words_host[0];
     if (logits_out) std::memcpy(logits_out, m->logits_host, C(m).vocab_size * sizeof(float));
     return 0;
@@ -1323,7 +1328,7 @@ int cheetah_hip_decode_greedy(cheetah_hip_model *m, uint32_t token, size_t offse
     CHIP_TRY(launch_set_step(m->step_dev, (int32_t)token, (int32_t)offset, m->stream));
     if (fused_fits(m, offset, steps)) CHIP_TRY(run_fused(m, offset, steps));
     else
-        for (size_t i = 0; i < steps; ++i) CHIP_TRY(launch_decode(m, offset + i));
+        for (size_t i = 0; i < steps; ++i) CHIP_TRY(launch_decode(m, offset + i, true));
     CHIP_CHECK(hipMemcpyAsync(tokens_out, m->hist_dev + offset + 1, steps * sizeof(uint32_t), hipMemcpyDeviceToHost,
                               m->stream));
     CHIP_CHECK(hipStreamSynchronize(m->stream));
@@ -1346,7 +1351,7 @@ int cheetah_hip_time_decode(cheetah_hip_model *m, uint32_t token, size_t offset,
     if (fused_fits(m, offset, steps)) {
         CHIP_TRY(run_fused(m, offset, steps));  // waits for the launch
     } else {
-        for (size_t i = 0; i < steps; ++i) CHIP_TRY(launch_decode(m, offset + i));
+        for (size_t i = 0; i < steps; ++i) CHIP_TRY(launch_decode(m, offset + i, true));
     }
     CHIP_CHECK(hipEventRecord(e1, m->stream));
     CHIP_CHECK(hipEventSynchronize(e1));
