@@ -718,7 +718,9 @@ __global__ __launch_bounds__(kThreads) void attn_combine_kernel(const float *par
 // registers and 16-bit transposing stores cost the rest. 512 rows on a 4K
 // prefix, 32 q / 8 KV heads of 128: 113 -> 89.8 us (316 -> 398 TFLOP/s, twice
 // that executed), with the same bits; rows direct to LDS and transposing reads
-// alone 97.5 us.
+// alone 97.5 us. At head_dim 64 (the small decoder's 16-block grids, where a
+// wave's chain of tiles is the time) both halves of a tile share one softmax
+// round: Qwen2-0.5B prefill of 512 tokens 7.47 -> 7.42 ms.
 //
 // Splits are absolute position ranges of `span` keys (fixed per model), so
 // every row's result depends only on its own position (the same bits however
@@ -825,6 +827,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     constexpr int RW = 32 / G, MV = RW * G;
     constexpr int KSTEPS = HD / 16, UT = HD / 32, KC = HD / 32;
     constexpr int CPR = HD / 8;  // 16-byte chunks per K row
+    constexpr int NH = HD == 64 ? 2 : 1;  // 32-position halves per softmax step
     // Two tiles each. K rows unpadded, chunk c of LDS row r stored at chunk
     // c ^ (r % CPR); V rows as they come, 64-byte segments swizzled by vseg.
     extern __shared__ __attribute__((aligned(16))) uint8_t smem_kv[];
@@ -932,38 +935,58 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             fetch(t0 + 64, page_next, b ^ 1);
             page_next = page_of(min(t0 + 128, last_tile));
         }
-        // Two halves of 32 positions, each: S^T, online softmax, O^T update.
+        // Steps of 32 NH positions, each: S^T, online softmax, O^T update. At
+        // head_dim 64 the registers hold both halves of the tile at once: two
+        // independent score chains and one softmax round for 64 keys.
         uint32_t vad[UT];
 #pragma unroll
         for (int u = 0; u < UT; ++u) vad[u] = vaddr[u] + b * TB;
-        auto half_tile = [&](auto half_index) {
-            constexpr int tt = decltype(half_index)::value;
-            f32x16 sacc = f32x16{};
+        auto step = [&](auto step_index) {
+            constexpr int p0 = 32 * NH * decltype(step_index)::value;
+            f32x16 sacc[NH];
+#pragma unroll
+            for (int x = 0; x < NH; ++x) sacc[x] = f32x16{};
 #pragma unroll
             for (int s = 0; s < KSTEPS; ++s) {
-                const int r = 32 * tt + n;
-                const bf16x8 ka =
-                    __builtin_bit_cast(bf16x8, *(const u32x4 *)(ks + b * TB + r * HD * 2 + 16 * ((2 * s + half) ^ (r % CPR))));
-                sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, qh[s], sacc, 0, 0, 0);
-                sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, ql[s], sacc, 0, 0, 0);
-            }
-            // The half's V^T fragments, while the score products drain.
-            bf16x8 va[2][UT];
-            read_vt<HD, (32 * tt) * HD * 2>(vad, va[0]);
-            read_vt<HD, (32 * tt + 16) * HD * 2>(vad, va[1]);
-            // Causal / split-end mask, only where the half reaches past a
-            // row's position or past the split (block-uniform test).
-            const int h0 = t0 + 32 * tt;
-            if (h0 + 31 > first_pos || h0 + 32 > end) {
+                bf16x8 ka[NH];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int p = h0 + krow_of(8 * (r >> 2) + 4 * half + (r & 3));
-                    if (p > my_pos || p >= end) sacc[r] = -INFINITY;
+                for (int x = 0; x < NH; ++x) {
+                    const int r = p0 + 32 * x + n;
+                    ka[x] = __builtin_bit_cast(
+                        bf16x8, *(const u32x4 *)(ks + b * TB + r * HD * 2 + 16 * ((2 * s + half) ^ (r % CPR))));
                 }
+#pragma unroll
+                for (int x = 0; x < NH; ++x)
+                    sacc[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[x], qh[s], sacc[x], 0, 0, 0);
+#pragma unroll
+                for (int x = 0; x < NH; ++x)
+                    sacc[x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[x], ql[s], sacc[x], 0, 0, 0);
+            }
+            // The step's V^T fragments, while the score products drain.
+            bf16x8 va[2 * NH][UT];
+            read_vt<HD, p0 * HD * 2>(vad, va[0]);
+            read_vt<HD, (p0 + 16) * HD * 2>(vad, va[1]);
+            if constexpr (NH == 2) {
+                read_vt<HD, (p0 + 32) * HD * 2>(vad, va[2]);
+                read_vt<HD, (p0 + 48) * HD * 2>(vad, va[3]);
+            }
+            // Causal / split-end mask, only where the step reaches past a
+            // row's position or past the split (block-uniform test).
+            const int h0 = t0 + p0;
+            if (h0 + 32 * NH - 1 > first_pos || h0 + 32 * NH > end) {
+#pragma unroll
+                for (int x = 0; x < NH; ++x)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int p = h0 + 32 * x + krow_of(8 * (r >> 2) + 4 * half + (r & 3));
+                        if (p > my_pos || p >= end) sacc[x][r] = -INFINITY;
+                    }
             }
             float tmax = -INFINITY;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, sacc[r]);
+            for (int x = 0; x < NH; ++x)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, sacc[x][r]);
             tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
             // Delayed rescaling: exponentials are taken against a reference
             // max m2 that is raised only when a score exceeds it by more than
@@ -984,19 +1007,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             const float mref = m2 == -INFINITY ? 0.f : m2;
             float tsum = 0.f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float pv = __builtin_amdgcn_exp2f(sacc[r] - mref);
-                sacc[r] = pv;
-                tsum += pv;
-            }
+            for (int x = 0; x < NH; ++x)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float pv = __builtin_amdgcn_exp2f(sacc[x][r] - mref);
+                    sacc[x][r] = pv;
+                    tsum += pv;
+                }
             tsum += __shfl_xor(tsum, 32, 64);
             l += tsum;
-            // O^T += V^T P^T over 2 steps of 16 positions.
+            // O^T += V^T P^T over steps of 16 positions.
 #pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
+            for (int s2 = 0; s2 < 2 * NH; ++s2) {
                 float pv[8];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) pv[j] = sacc[8 * s2 + j];
+                for (int j = 0; j < 8; ++j) pv[j] = sacc[s2 >> 1][8 * (s2 & 1) + j];
                 bf16x8 bh, bl;
                 split8(pv, bh, bl);
 #pragma unroll
@@ -1006,8 +1031,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
                 }
             }
         };
-        half_tile(std::integral_constant<int, 0>{});
-        half_tile(std::integral_constant<int, 1>{});
+        step(std::integral_constant<int, 0>{});
+        if constexpr (NH == 1) step(std::integral_constant<int, 1>{});
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         if (more && t0 + 128 > end) clear_v(t0 + 64, b ^ 1);
         __syncthreads();
