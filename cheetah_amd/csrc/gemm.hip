@@ -45,7 +45,8 @@ struct GArgs {
     size_t stride;
     int N, K, M;  // N = weight rows, K = cols, M = tokens
     const float *x;
-    const uint16_t *xh, *xl;  // x pre-split into hi / lo BF16 halves, [M][K] (or null)
+    const uint16_t *xh, *xl;  // x pre-split into hi / lo BF16 halves, [M][xs] (or null)
+    int xs;                   // elements between rows of xh / xl (K, or K padded with zeros)
     const float *bias;
     float *y, *residual;
     uint16_t *yh, *yl;  // SwiGLU: the output also as BF16 halves (or null)
@@ -550,10 +551,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_ring_kernel(GArgs a, int
     const int hc = (a.nchunks + 1) / 2;
     const int kbeg = split == 1 ? blockIdx.z * a.chunk : split == 2 && blockIdx.z ? hc * a.chunk : 0;
     const int kend = split == 1 ? min(a.K, kbeg + a.chunk) : split == 2 && !blockIdx.z ? min(a.K, hc * a.chunk) : a.K;
-    const int nst = (kend - kbeg) / BK;
+    const int nst = (kend - kbeg + BK - 1) / BK;  // a part stage only against zero-padded x (Q8/Q4)
 
-    const __amdgpu_buffer_rsrc_t rxh = __builtin_amdgcn_make_buffer_rsrc((void *)a.xh, (short)0, a.M * a.K * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rxl = __builtin_amdgcn_make_buffer_rsrc((void *)a.xl, (short)0, a.M * a.K * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rxh = __builtin_amdgcn_make_buffer_rsrc((void *)a.xh, (short)0, a.M * a.xs * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rxl = __builtin_amdgcn_make_buffer_rsrc((void *)a.xl, (short)0, a.M * a.xs * 2, 0x00020000);
     const int wbytes = (int)((size_t)a.N * a.stride);
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)a.w, (short)0, wbytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rw2 =
@@ -564,7 +565,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_ring_kernel(GArgs a, int
     for (int i = 0; i < NIX / WV; ++i) {
         const int q = wave + WV * i, r = 16 * q + (lane >> 2);
         const int m = min(m0 + r, a.M - 1);  // rows past M feed only unstored outputs
-        xoff[i] = (m * a.K + 8 * swz(r, lane & 3)) * 2;
+        xoff[i] = (m * a.xs + 8 * swz(r, lane & 3)) * 2;
     }
     // Weight copy q covers rows RPC q .. RPC q + RPC - 1 of the tile; with
     // DUAL the first half of the copies reads the gate matrix, the rest up.
@@ -949,13 +950,15 @@ int launch_ring_plan(GArgs &a, const RingPlan &p, hipStream_t s) {
 
 template <int FMT>
 int launch_fmt(GArgs a, bool dual, size_t ws_floats, hipStream_t s, bool &split_out, int &stored_out) {
-    // Pre-split x with K a multiple of the stage and 32-bit buffer offsets:
-    // the ring kernel (weights copied 16 bytes at a time, Q4 and unaligned Q8 4).
+    // Pre-split x with K a multiple of the stage (Q8/Q4: or x padded to one
+    // with zeros, which whatever codes follow the row's meet; a BF16 row's
+    // neighbour could hold a NaN) and 32-bit buffer offsets: the ring kernel (weights copied 16 bytes at a time, Q4 and unaligned Q8 4).
     const int galign = FMT == FMT_BF16 ? 16 : 4;
-    const bool ring = a.xh && a.K % BK == 0 && a.stride % galign == 0 &&
+    const int kpad = (a.K + BK - 1) / BK * BK;
+    const bool ring = a.xh && (FMT == FMT_BF16 ? a.K : a.xs) % BK == 0 && a.xs >= kpad && a.stride % galign == 0 &&
                       ((uintptr_t)a.w % galign) == 0 &&
                       (!dual || (((uintptr_t)a.w | (uintptr_t)a.w2 | a.stride) % (FMT == FMT_Q4 ? 4 : 16)) == 0) &&
-                      (size_t)a.M * a.K * 2 < (1ull << 31) && (size_t)a.N * a.stride < (1ull << 31);
+                      (size_t)a.M * a.xs * 2 < (1ull << 31) && (size_t)a.N * a.stride < (1ull << 31);
     if (ring) {
         const RingPlan p = ring_plan(FMT, dual, a.N, a.K, a.M, a.ws ? ws_floats : 0);
         split_out = p.split != 0;
@@ -967,6 +970,7 @@ int launch_fmt(GArgs a, bool dual, size_t ws_floats, hipStream_t s, bool &split_
     }
     // Otherwise (K not a multiple of the stage, x not pre-split, or operands
     // beyond the buffer loads' 32-bit offsets): the register-staged kernel.
+    if (a.xs != a.K) a.xh = a.xl = nullptr;
     // Many tiles: fold in registers. Few tiles: split-K over the chunks when
     // the workspace holds them.
     const long n_tiles = (a.N + BN - 1) / BN;
@@ -1006,7 +1010,44 @@ __global__ __launch_bounds__(kThreads) void split_bf16_kernel(const float *x, si
     }
 }
 
+// The same for rows of K elements into rows of ks (a multiple of 4), zeros
+// past K.
+__global__ __launch_bounds__(kThreads) void split_bf16_rows_kernel(const float *x, size_t n, int K, int ks,
+                                                                   uint16_t *xh, uint16_t *xl) {
+    const size_t i = ((size_t)blockIdx.x * kThreads + threadIdx.x) * 4;
+    if (i >= n * ks) return;
+    const size_t row = i / ks;
+    const int c = (int)(i % ks);
+    uint16_t h[4], l[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float v = c + q < K ? x[row * K + c + q] : 0.f;
+        const __bf16 hb = (__bf16)v;
+        h[q] = __builtin_bit_cast(uint16_t, hb);
+        l[q] = __builtin_bit_cast(uint16_t, (__bf16)(v - (float)hb));
+    }
+    *(uint2 *)(xh + i) = make_uint2(pack2(h[0], h[1]), pack2(h[2], h[3]));
+    *(uint2 *)(xl + i) = make_uint2(pack2(l[0], l[1]), pack2(l[2], l[3]));
+}
+
 }  // namespace
+
+size_t gemm_half_stride(int fmt, size_t cols) { return fmt == FMT_BF16 ? cols : (cols + BK - 1) / BK * BK; }
+
+int launch_split_bf16_rows(const float *x, size_t n, size_t cols, size_t stride, uint16_t *xh, uint16_t *xl,
+                           hipStream_t s) {
+    if (stride == cols) return launch_split_bf16(x, n * cols, xh, xl, s);
+    if (n == 0) return 0;
+    if (!x || !xh || !xl || stride < cols || stride % 4 || stride > (size_t)INT32_MAX || ((uintptr_t)xh % 8) ||
+        ((uintptr_t)xl % 8))
+        return fail("HIP backend: split needs rows padded to a multiple of 4 and 8-byte aligned halves.");
+    const size_t blocks = (n * stride / 4 + kThreads - 1) / kThreads;
+    if (blocks > (size_t)INT32_MAX) return fail("HIP backend: split shape too large.");
+    hipLaunchKernelGGL(split_bf16_rows_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, s, x, n, (int)cols,
+                       (int)stride, xh, xl);
+    CHIP_CHECK(hipGetLastError());
+    return 0;
+}
 
 int launch_split_bf16(const float *x, size_t n, uint16_t *xh, uint16_t *xl, hipStream_t s) {
     if (n == 0) return 0;
@@ -1037,7 +1078,7 @@ size_t gemm_workspace_floats(int fmt, size_t N, size_t K, size_t M, bool dual) {
     const int chunk = gemm_chunk_depth((int)K);
     const size_t nchunks = (K + chunk - 1) / chunk, tiles = (N + BN - 1) / BN * ((M + 63) / 64);
     const size_t staged = nchunks > 1 && tiles < (size_t)device_cus() ? nchunks * M * N * (dual ? 2 : 1) : 0;
-    return K % BK ? staged : std::max(staged, ring_plan(fmt, dual, (int)N, (int)K, (int)M, SIZE_MAX).ws_floats);
+    return K % BK && fmt == FMT_BF16 ? staged : std::max(staged, ring_plan(fmt, dual, (int)N, (int)K, (int)M, SIZE_MAX).ws_floats);
 }
 
 size_t gemm_split_workspace_floats(int fmt, size_t N, size_t K, size_t m_max, bool dual) {
@@ -1053,9 +1094,10 @@ int launch_gemm(const GemmJob &job, hipStream_t s) {
     if (job.n == 0) return 0;
     // Pre-split halves are used when every 8-element chunk is 16-byte aligned;
     // x itself is then not read.
-    const bool pre = job.xh && job.xl && gemm_takes_halves(w.cols) && ((uintptr_t)job.xh % 16) == 0 &&
-                     ((uintptr_t)job.xl % 16) == 0;
-    if (!w.base || (!job.x && !pre) || w.rows == 0 || w.cols == 0)
+    const size_t xs = job.x_stride ? job.x_stride : w.cols;
+    if (xs < w.cols || xs > (size_t)INT32_MAX) return fail("HIP backend: gemm input rows are too short or too long.");
+    const bool pre = job.xh && job.xl && xs % 8 == 0 && ((uintptr_t)job.xh % 16) == 0 && ((uintptr_t)job.xl % 16) == 0;
+    if (!w.base || (!job.x && !(pre && xs == w.cols)) || w.rows == 0 || w.cols == 0)
         return fail("HIP backend: gemm needs a weight and an input.");
     if (w.rows > (size_t)INT32_MAX || w.cols > (size_t)INT32_MAX || job.n > 65535u * 64u)
         return fail("HIP backend: gemm shape too large.");
@@ -1086,6 +1128,7 @@ int launch_gemm(const GemmJob &job, hipStream_t s) {
     a.nchunks = (a.K + a.chunk - 1) / a.chunk;
     a.ws = job.ws;
     a.vec_x = (a.K % 4) == 0 && ((uintptr_t)job.x % 16) == 0;
+    a.xs = (int)xs;
     a.xh = pre ? job.xh : nullptr;
     a.xl = pre ? job.xl : nullptr;
     const uintptr_t p1 = (uintptr_t)a.w, p2 = dual ? (uintptr_t)a.w2 : p1;

@@ -61,6 +61,10 @@ struct GemmJob {
     // (the same bits).
     // x may be null where gemm_takes_halves(cols).
     const uint16_t *xh = nullptr, *xl = nullptr;
+    // Elements between rows of xh / xl; 0 = cols. Q8/Q4 matrices whose column
+    // count is no multiple of 32 run on the ring kernel when the halves' rows
+    // are padded to gemm_half_stride with zeros (launch_split_bf16_rows).
+    size_t x_stride = 0;
     // EPI_SWIGLU only, optional: the output also as BF16 halves ([n][rows]
     // each, the bits launch_split_bf16 would give), for the next GEMM; y may
     // then be null.
@@ -76,6 +80,10 @@ int launch_gemm(const GemmJob &job, hipStream_t stream);
 // Whether a GEMM over K columns given xh / xl reads them and not x.
 bool gemm_takes_halves(size_t K);
 int launch_split_bf16(const float *x, size_t n, uint16_t *xh, uint16_t *xl, hipStream_t s);
+// n rows of `cols` into rows of `stride` (zeros past cols).
+int launch_split_bf16_rows(const float *x, size_t n, size_t cols, size_t stride, uint16_t *xh, uint16_t *xl,
+                           hipStream_t s);
+size_t gemm_half_stride(int fmt, size_t cols);
 int gemm_chunk_depth(int K);
 // Split-K scratch a GEMM of M tokens uses; with less it runs another split
 // or none (the same bits).
