@@ -161,11 +161,12 @@ def test_gemm_bits_independent_of_token_count(hip, fmt):
 
 @pytest.mark.parametrize("fmt", ["bf16", "q8", "q4"])
 @pytest.mark.parametrize("rows,cols", [(1001, 64), (515, 896), (4097, 4096), (14336, 1024), (130, 33), (259, 1001),
-                                       (4096, 1009)])
+                                       (4096, 1009), (9001, 2048)])
 def test_gemm_tile_edges_give_the_same_bits(hip, oracle, fmt, rows, cols):
     """Token counts and row counts around the edges of the 64 / 128-token and
     128 / 256-row tiles, odd row counts (Q8 payloads only 4-byte aligned) and
-    every K split the sizes choose, with column counts that end inside a
+    every K split the sizes choose (9001 x 2048 at 1,030 tokens: full rounds
+    of large tiles, then the rest on smaller ones), with column counts that end inside a
     32-column stage (Q8/Q4 on zero-padded input halves): a token's outputs are the same bits in
     every call, and the oracle's within the hi/lo input split (2^-17 per
     product; 1e-5 of the largest output)."""
