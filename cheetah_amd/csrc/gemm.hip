@@ -949,9 +949,8 @@ RingPlan ring_plan(int fmt, bool dual, int N, int K, int M, size_t ws_floats) {
     const float us_mid = (fmt == FMT_BF16 ? mid.us_bf16 : mid.us_quant) * (float)K / 1024.f;
     const int bno = dual ? big.bn / 2 : big.bn, bno_mid = dual ? mid.bn / 2 : mid.bn;
     const long m_tiles = (M + big.bm - 1) / big.bm, n_tiles = (N + bno - 1) / bno;
-    for (long rounds = 1; rounds * cus < m_tiles * n_tiles; ++rounds) {
-        const long head = rounds * cus / m_tiles;
-        if (head == 0 || head * bno >= N) continue;
+    const long rounds = m_tiles * n_tiles / cus, head = rounds * cus / m_tiles;
+    if (head > 0 && head * bno < N) {
         const long rest = (N - head * bno + bno_mid - 1) / bno_mid * m_tiles;
         const float est = (float)rounds * us_big + (float)((rest + cus - 1) / cus) * us_mid + 8.f;
         if (est < best_us) {
