@@ -95,6 +95,35 @@ def test_tiny_greedy_32_steps_token_exact(hip, oracle, shape, kv):
     assert [first] + rest.tolist() == ref_tokens
 
 
+@pytest.mark.parametrize("quant", [None, "q4"])
+@pytest.mark.parametrize("shape", TINY, ids=lambda s: s.name)
+def test_mixed_forward_calls_agree_with_device_greedy(hip, shape, quant):
+    """forward (no sampling), forward_greedy with and without logits and
+    decode_greedy in turn on one cache: the same tokens as decode_greedy alone
+    and the same logit bits from either forward, on the persistent kernel and
+    the decode graphs; the logits reach the host whole (an odd vocabulary ends
+    inside a vector store)."""
+    from cheetah_amd.workloads import greedy_token
+
+    g = hip.HipForward(shape, weights(shape), quant=quant, kv_capacity=256, max_chunk_rows=32)
+    prompt = synth.make_tokens(shape.vocab_size, 20, seed=4)
+    first, logits = g.forward_greedy(prompt, 0, want_logits=True)
+    assert first == greedy_token(logits)
+    want = [first] + g.decode_greedy(first, 20, 8).tolist()
+    g.clear_cache()
+    assert np.array_equal(bits(g.forward(prompt, 0)), bits(logits))
+    got = [first]
+    got.append(greedy_token(g.forward(np.array(got[-1:], np.uint32), 20)))
+    got.append(g.forward_greedy(np.array(got[-1:], np.uint32), 21))
+    got += g.decode_greedy(got[-1], 22, 2).tolist()
+    tok, lg = g.forward_greedy(np.array(got[-1:], np.uint32), 24, want_logits=True)
+    assert tok == greedy_token(lg)
+    got.append(tok)
+    got.append(greedy_token(g.forward(np.array(got[-1:], np.uint32), 25)))
+    got += g.decode_greedy(got[-1], 26, 2).tolist()
+    assert got == want
+
+
 @pytest.mark.parametrize("shape", TINY, ids=lambda s: s.name)
 def test_f32_kv_prefill_attention_tile_and_span_edges(hip, oracle, shape):
     """f32-cache prefill attention at the edges of its 64-key tiles, 256-key
