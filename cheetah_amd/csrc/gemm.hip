@@ -468,6 +468,9 @@ __global__ __launch_bounds__(kThreads) void gemm_reduce_kernel(GArgs a);
 // s_waitcnt immediate waiting until at most n vector-memory ops are pending.
 constexpr int vm_wait_imm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
 
+// Stages of the deeper BF16 ring of 4-wave blocks (launch_ring_plan).
+constexpr int kDeepStages = 5;
+
 // Raw weight bytes per row and 32-column stage.
 template <int FMT>
 constexpr int w_row_bytes() { return FMT == FMT_BF16 ? 64 : FMT == FMT_Q8 ? 32 : 16; }
@@ -705,7 +708,11 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_ring_kernel(GArgs a, int
 #pragma unroll
         for (int j = 0; j < 2; ++j) tot[i][j] = f32x16{};
 
-    constexpr int DH = D / 2 + D % 2;  // copies issued in a stage's second k-step
+    // Copies issued in a stage's second k-step, the rest in the next stage's
+    // first: half of them; on the deep BF16 ring, whose time is the weight
+    // stream and not the MFMAs, all (18944 x 3584 at 2 tokens 41.7 -> 40.8 us,
+    // 10112 x 2304 at 16 23.8 -> 21.7; Q8/Q4 3 % slower at small sizes).
+    constexpr int DH = !CONV && NS >= kDeepStages ? D : D / 2 + D % 2;
 #pragma unroll
     for (int st = 0; st < NS - 1; ++st)
 #pragma unroll
@@ -876,8 +883,9 @@ int launch_mt(const GArgs &a, bool split, hipStream_t s) {
     return 0;
 }
 
-// Ring stages by format: the 4-wave tile keeps two blocks per CU (64 to 76 KB
-// each), the others one.
+// Ring stages by format: the 4-wave tile keeps two blocks per CU (64 to 80 KB
+// each), the others one. BF16 blocks of 4 waves have a second, deeper ring
+// (launch_ring_plan).
 template <int FMT>
 constexpr int ring_stages() { return FMT == FMT_BF16 ? 4 : 5; }
 
@@ -972,7 +980,22 @@ int launch_ring_plan(GArgs &a, const RingPlan &p, hipStream_t s) {
         a.n_first = p.head_tiles * (DUAL ? 128 : 256);
     }
     switch (p.tile) {
-        case TILE_64x128: return launch_ring<FMT, DUAL, 1, 2, 2, NS, QG>(a, p.split, s);
+        case TILE_64x128:
+            // BF16 at few tokens is the weight stream: five stages, two of them
+            // in flight at every wait (with four one: 4864 x 14336 at 16 tokens
+            // 51.0 -> 43.2 us, 896 x 18944 at 4 21.6 -> 18.2). Four where a
+            // split leaves nine stages or fewer a block and one to four blocks
+            // a CU, or K is six or fewer, so that a deeper fill shows (4096 x
+            // 4096 at 16 tokens 15.5 against 16.3, 6144 x 4096 at 37 27.6
+            // against 28.4, 640 x 128 at 4 6.9 against 7.2).
+            if constexpr (FMT == FMT_BF16) {
+                constexpr int BNO = DUAL ? 64 : 128;
+                const long blocks = (long)((a.N + BNO - 1) / BNO) * ((a.M + 63) / 64) * p.nstored, cus = device_cus();
+                const bool short_blocks = a.K <= 6 * BK || (p.split == 1 && a.chunk <= 9 * BK && blocks > cus &&
+                                                            blocks <= 4 * cus);
+                if (!short_blocks) return launch_ring<FMT, DUAL, 1, 2, 2, kDeepStages, QG>(a, p.split, s);
+            }
+            return launch_ring<FMT, DUAL, 1, 2, 2, NS, QG>(a, p.split, s);
         case TILE_128x128: return launch_ring<FMT, DUAL, 1, 4, 2, NS, QG>(a, p.split, s);
         default: return launch_ring<FMT, DUAL, 2, 2, 4, NS, QG>(a, p.split, s);
     }

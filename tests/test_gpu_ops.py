@@ -188,6 +188,31 @@ def test_gemm_tile_edges_give_the_same_bits(hip, oracle, fmt, rows, cols):
     assert rel_err(full[sel], ref) < 1e-5
 
 
+@pytest.mark.parametrize("fmt", ["bf16", "q8", "q4"])
+@pytest.mark.parametrize("rows,cols", [(20000, 2048), (4096, 2304)])
+def test_gemm_few_tokens_give_the_same_bits(hip, oracle, fmt, rows, cols):
+    """The weight stream of few tokens: BF16 on the five-stage ring (20000 x 2048, over four
+    blocks a CU) and on the four-stage one (4096 x 2304, one to four): the same
+    bits at every token count, and the oracle's within the hi/lo input split
+    (2^-17 per product; 1e-5 of the largest output)."""
+    rng = np.random.default_rng(rows + 3 * cols)
+    x = rng.standard_normal((130, cols)).astype(np.float32)
+    if fmt == "bf16":
+        w = synth.f32_to_bf16(rng.standard_normal((rows, cols)).astype(np.float32))
+        wd = hip.DeviceBuffer.from_array(w)
+    else:
+        buf = random_quant(rng, fmt, rows, cols)
+        wd = hip.DeviceBuffer.from_array(buf)
+    full = np.ascontiguousarray(hip.gemm(wd, fmt, rows, cols, x))
+    for n in (1, 8, 9, 37, 64, 65):
+        got = np.ascontiguousarray(hip.gemm(wd, fmt, rows, cols, x[:n]))
+        assert np.array_equal(got.view(np.uint32), full[:n].view(np.uint32)), n
+    sel = np.array([0, 36, 64, 129])
+    xs = np.ascontiguousarray(x[sel])
+    ref = oracle.gemm_bf16(w, xs) if fmt == "bf16" else oracle.gemm_quant(buf, rows, cols, xs, fmt)
+    assert rel_err(full[sel], ref) < 1e-5
+
+
 def _attn_case(rng, q_heads, kv_heads, hd, ctx, rows):
     k = synth.f32_to_bf16(rng.standard_normal((ctx, kv_heads, hd)).astype(np.float32))
     v = synth.f32_to_bf16(rng.standard_normal((ctx, kv_heads, hd)).astype(np.float32))
