@@ -903,25 +903,23 @@ struct RingPlan {
 // The plan with the least estimated time of those whose stored sums fit
 // ws_floats. The estimate, in us: rounds of the tile's blocks (one per CU, two
 // for the 4-wave tile) times the time of 1,024 columns of a block in a full
-// round (with no more blocks than CUs, of a block alone), and 3 to fill and
-// drain; a split adds a launch or a longer reader (2) and its sums' write and
-// read at 4.5 TB/s. Measured per 1,024 columns: 128 x 256 tiles 31 us (BF16)
-// and 34 (Q8/Q4) on 256 CUs, 128 x 128 18 to 20, 64 x 128 24 (27), alone 16
-// (18 to 20). Examples (BF16, x split included), chosen against the next best:
-// 14336 x 4096 at 512 tokens 128 x 256 unsplit 119 us (128 x 128 152); 4096 x
-// 14336 at 512 128 x 128 halves 152 (128 x 256 halves 175); 6144 x 4096 at 512
-// 128 x 256 halves 69 (128 x 128 unsplit 78); 4096 x 4096 at 256 128 x 128
-// halves 45 (64 x 128 per chunk 60), at 192 64 x 128 halves 39 (128 x 128
-// halves 41); 1152 x 896 at 128 64 x 128 per chunk 11.9 (128 x 128 13.0); 3584
-// x 18944 at 128 128 x 128 per chunk 67 (64 x 128 80).
+// round (with no more blocks than CUs, of a block alone), and a fixed time per
+// tile, with and without a split; a split adds its sums' write and read at 3.5
+// TB/s, an unsplit wave's epilogue takes 3 us for 32 rows. The figures are
+// those with which the choice came closest to the best of every tile and
+// split, timed at 1,772 sizes of 64 to 20000 rows, 64 to 18944 columns and 2 to
+// 2,048 tokens in the three formats: 0.3 % behind it on average (1.8 % with one
+// fixed time for all tiles, unsplit less than split: 2240 x 128 Q8 at 37 tokens
+// then ran 64 x 128 unsplit, 11.9 us against 9.5 split).
 RingPlan ring_plan(int fmt, bool dual, int N, int K, int M, size_t ws_floats) {
     static constexpr struct {
         int bm, bn, per_cu;
         float us_bf16, us_quant;    // a full round
         float low_bf16, low_quant;  // no more blocks than CUs
-    } kTiles[] = {{64, 128, 2, 24.f, 27.f, 16.f, 19.f},
-                  {128, 128, 1, 19.f, 19.f, 19.f, 19.f},
-                  {128, 256, 1, 30.f, 34.f, 30.f, 34.f}};
+        float fixed, fixed_split;   // without and with a split
+    } kTiles[] = {{64, 128, 2, 26.f, 29.f, 13.f, 17.5f, 3.f, 2.f},
+                  {128, 128, 1, 21.f, 22.f, 17.5f, 19.f, 4.f, 4.f},
+                  {128, 256, 1, 30.f, 34.f, 25.5f, 32.5f, 5.5f, 4.5f}};
     const int chunk = gemm_chunk_depth(K), nchunks = (K + chunk - 1) / chunk;
     const long cus = device_cus();
     const float mn = (float)M * (float)N;
@@ -940,8 +938,13 @@ RingPlan ring_plan(int fmt, bool dual, int N, int K, int M, size_t ws_floats) {
             const long slots = cus * kTiles[t].per_cu, rounds = (tiles * parts + slots - 1) / slots;
             const float us = tiles * parts > cus ? bf ? kTiles[t].us_bf16 : kTiles[t].us_quant
                                                  : bf ? kTiles[t].low_bf16 : kTiles[t].low_quant;
-            float est = (float)rounds * (float)depth / 1024.f * us + 3.f;
-            if (split) est += 2.f + 8.f * (float)parts * (dual ? 2.f : 1.f) * mn / 4.5e6f;
+            float est = (float)rounds * (float)depth / 1024.f * us + (split ? kTiles[t].fixed_split : kTiles[t].fixed);
+            if (split) {
+                est += 8.f * (float)parts * (dual ? 2.f : 1.f) * mn / 3.5e6f;
+            } else {
+                const int rows = t == TILE_128x256 ? 64 : 32;  // of a wave
+                est -= 3.f * (float)(rows - std::min(M, rows)) / 32.f;
+            }
             if (best_us == 0.f || est < best_us) {
                 best_us = est;
                 best = RingPlan{t, split, parts, need, 0};
@@ -960,7 +963,7 @@ RingPlan ring_plan(int fmt, bool dual, int N, int K, int M, size_t ws_floats) {
     const long rounds = m_tiles * n_tiles / cus, head = rounds * cus / m_tiles;
     if (head > 0 && head * bno < N) {
         const long rest = (N - head * bno + bno_mid - 1) / bno_mid * m_tiles;
-        const float est = (float)rounds * us_big + (float)((rest + cus - 1) / cus) * us_mid + 8.f;
+        const float est = (float)rounds * us_big + (float)((rest + cus - 1) / cus) * us_mid + 11.f;
         if (est < best_us) {
             best_us = est;
             best = RingPlan{TILE_128x128, 0, 1, 0, (int)head};

@@ -189,9 +189,10 @@ def test_gemm_tile_edges_give_the_same_bits(hip, oracle, fmt, rows, cols):
 
 
 @pytest.mark.parametrize("fmt", ["bf16", "q8", "q4"])
-@pytest.mark.parametrize("rows,cols", [(20000, 2048), (4096, 2304)])
-def test_gemm_few_tokens_give_the_same_bits(hip, oracle, fmt, rows, cols):
-    """The weight stream of few tokens: BF16 on the five-stage ring (20000 x 2048, over four
+@pytest.mark.parametrize("rows,cols", [(2240, 128), (640, 160), (20000, 2048), (4096, 2304)])
+def test_gemm_few_tokens_and_few_columns_give_the_same_bits(hip, oracle, fmt, rows, cols):
+    """Few columns (unsplit or per chunk by the token count) and the weight
+    stream of few tokens: BF16 on the five-stage ring (20000 x 2048, over four
     blocks a CU) and on the four-stage one (4096 x 2304, one to four): the same
     bits at every token count, and the oracle's within the hi/lo input split
     (2^-17 per product; 1e-5 of the largest output)."""
