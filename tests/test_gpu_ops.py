@@ -248,6 +248,26 @@ def test_attention_decode_around_the_one_block_limit(hip, oracle, q_heads, kv_he
     assert rel_err(got, ref) < 2e-5
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("ctx", [65536, 65537, 131072])
+def test_attention_prefill_merges_more_than_64_splits(hip, hd, ctx):
+    """Two rows at the end of a long context: 64, 65 and 128 splits of 1,024
+    keys, two a lane in the merge, against the same in 64 bits. Queries and
+    probabilities are two BF16 halves (2^-17 per product, averaged over the keys
+    as the output is): 2e-5 of the largest output."""
+    rng = np.random.default_rng(ctx + hd)
+    k, v, q = _attn_case(rng, 2, 1, hd, ctx, 2)
+    kp, vp, table = hip.paged_kv(k, v, seed=7)
+    got = hip.attention(q, kp, vp, table, 2, 2, ctx - 2).reshape(2, 2, hd)
+    kf, vf = (synth.bf16_to_f32(t)[:, 0].astype(np.float64) for t in (k, v))
+    for row in range(2):
+        n = ctx - 1 + row
+        s = q[row].reshape(2, hd).astype(np.float64) @ kf[:n].T / np.sqrt(hd)
+        w = np.exp(s - s.max(axis=1, keepdims=True))
+        ref = w @ vf[:n] / w.sum(axis=1, keepdims=True)
+        assert rel_err(got[row], ref) < 2e-5, row
+
+
 @pytest.mark.parametrize("q_heads,kv_heads,hd,offset,rows", [(14, 2, 64, 0, 37), (32, 8, 128, 100, 70),
                                                             (28, 4, 128, 4000, 9)])
 def test_attention_prefill_rows_match_oracle(hip, oracle, q_heads, kv_heads, hd, offset, rows):
