@@ -1096,9 +1096,25 @@ constexpr int kF32LdV = 64 + 8;  // transposed V row: 64 positions + 16 bytes
 template <int HD>
 constexpr size_t prefill_f32_lds_bytes() { return (size_t)3 * 2 * (64 * HD + HD * kF32LdV); }
 
-template <int HD, int G>
+// One more part of a row's softmax (maximum m, weight sum l, values o) folded
+// into the running one (M, L, O), parts in order; a part without a key (m =
+// -inf) changes nothing. The factors of a part, for every value of the row.
+__device__ __forceinline__ void fold_factors(float m, float &M, float &alpha, float &beta) {
+    const float mn = fmaxf(M, m);
+    const bool any = m != -INFINITY;
+    alpha = any ? __builtin_amdgcn_exp2f(M - mn) : 1.f;
+    beta = any ? __builtin_amdgcn_exp2f(m - mn) : 0.f;
+    M = mn;
+}
+__device__ __forceinline__ float fold_value(float O, float o, float alpha, float beta) {
+    return fmaf(beta, o, O * alpha);
+}
+
+// FOLD: the block's split is longer than `sub` keys; its parts of `sub` keys
+// are folded in registers, in order (launch_prefill_f32).
+template <int HD, int G, bool FOLD>
 __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_kernel(AttnArgs a, int rows, int S,
-                                                                                     int span) {
+                                                                                     int span, int sub) {
     constexpr int RW = 32 / G, MV = RW * G;
     constexpr int LDV = kF32LdV;
     constexpr int KSTEPS = HD / 16, UT = HD / 32;
@@ -1204,6 +1220,10 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
 #pragma unroll
     for (int u = 0; u < UT; ++u) oacc[u] = f32x16{};
     float m2 = -INFINITY, l = 0.f;
+    f32x16 osum[FOLD ? UT : 1];
+#pragma unroll
+    for (int u = 0; u < (FOLD ? UT : 1); ++u) osum[u] = f32x16{};
+    float msum = -INFINITY, lsum = 0.f;
     for (int t0 = start; t0 < end; t0 += 64) {
         __syncthreads();  // the previous tile's reads are done
         stage();
@@ -1285,9 +1305,30 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
                 }
             }
         }
+        if constexpr (FOLD) {
+            if ((t0 + 64) % sub == 0 || t0 + 64 >= end) {
+                // A part without a key of the row may hold NaN (its -inf maximum
+                // rescaled with its neighbours'): left out, as the merge does.
+                const bool any = m2 != -INFINITY;
+                float alpha, beta;
+                fold_factors(m2, msum, alpha, beta);
+                lsum = any ? fold_value(lsum, l, alpha, beta) : lsum;
+#pragma unroll
+                for (int u = 0; u < UT; ++u) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        osum[u][r] = any ? fold_value(osum[u][r], oacc[u][r], alpha, beta) : osum[u][r];
+                    oacc[u] = f32x16{};
+                }
+                m2 = -INFINITY;
+                l = 0.f;
+            }
+        }
     }
     if (!rvalid) return;
-    store_prefill_rows<HD>(a, oacc, m2, l, part, (size_t)row * a.q_heads * HD + (size_t)head * HD, S, half);
+    const size_t ob = (size_t)row * a.q_heads * HD + (size_t)head * HD;
+    if constexpr (FOLD) store_prefill_rows<HD>(a, osum, msum, lsum, part, ob, S, half);
+    else store_prefill_rows<HD>(a, oacc, m2, l, part, ob, S, half);
 }
 
 // Merges the splits of one (row, q head) of attn_prefill_kernel in split
@@ -1336,39 +1377,185 @@ __global__ __launch_bounds__(kThreads) void attn_merge2_kernel(const float *part
     }
 }
 
+template <int HD>
+int launch_merge2(const AttnJob &j, const AttnArgs &a, int S, hipStream_t s) {
+    if (S <= 1) return 0;
+    const int items = (int)j.rows * j.q_heads;
+    hipLaunchKernelGGL((attn_merge2_kernel<HD>), dim3((items + 3) / 4), dim3(kThreads), 0, s, a.part, S, j.q_heads,
+                       items, a.out, a.out_hi, a.out_lo);
+    CHIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+// Most parts of attn_merge_parts_kernel (their factors sit in LDS).
+constexpr int kMaxParts = 256;
+
+// Merges the parts of one (row, q head) of an f32 prefill, one wave per (row,
+// head): the `per` parts of each split folded in order, as the FOLD kernel
+// does, then the splits as attn_merge2_kernel does (one lane per split): the
+// bits of the FOLD kernel and attn_merge2_kernel.
+template <int HD>
+__global__ __launch_bounds__(kThreads) void attn_merge_parts_kernel(const float *part, int parts, int per, int q_heads,
+                                                                   int items, float *out, uint16_t *out_hi,
+                                                                   uint16_t *out_lo) {
+    __shared__ float2 s_f[kThreads / 64][kMaxParts];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int item = blockIdx.x * (kThreads / 64) + wave;
+    if (item >= items) return;
+    const float *p = part + (size_t)item * (size_t)parts * (HD + 2);
+    const int S = (parts + per - 1) / per;
+    // Lane g: the maximum and the weight sum of split g, its parts' factors.
+    float m = -INFINITY, l = 0.f;
+    if (lane < S) {
+        for (int i = lane * per; i < min(lane * per + per, parts); ++i) {
+            const float mi = p[(size_t)i * (HD + 2) + HD];
+            const float li = mi == -INFINITY ? 0.f : p[(size_t)i * (HD + 2) + HD + 1];
+            float alpha, beta;
+            fold_factors(mi, m, alpha, beta);
+            l = fold_value(l, li, alpha, beta);
+            s_f[wave][i] = make_float2(alpha, mi == -INFINITY ? -1.f : beta);  // -1: the part holds no values
+        }
+    }
+    // The factors are read by the whole wave: its LDS operations run in order.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const float M = wave_max(m);
+    const float w = m == -INFINITY ? 0.f : exp2f(m - M);
+    const float L = wave_sum(w != 0.f ? w * l : 0.f);
+    const float inv = 1.0f / L;
+    constexpr int DPL = HD / 64, BATCH = 16;  // dims per lane; parts loaded per round trip
+    float o[DPL], t[DPL];
+#pragma unroll
+    for (int k = 0; k < DPL; ++k) o[k] = t[k] = 0.f;
+    for (int i0 = 0; i0 < parts; i0 += BATCH) {
+        float v[BATCH][DPL];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const int q = min(i0 + i, parts - 1);
+#pragma unroll
+            for (int k = 0; k < DPL; ++k) v[i][k] = p[(size_t)q * (HD + 2) + lane + 64 * k];
+        }
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const int q = i0 + i;
+            if (q < parts) {
+                const float2 f = s_f[wave][q];
+#pragma unroll
+                for (int k = 0; k < DPL; ++k)
+                    t[k] = f.y < 0.f ? t[k] : fold_value(t[k], v[i][k], f.x, f.y);
+                if ((q + 1) % per == 0 || q + 1 == parts) {
+                    const float ws = __shfl(w, q / per, 64);
+#pragma unroll
+                    for (int k = 0; k < DPL; ++k) {
+                        if (ws != 0.f) o[k] = fmaf(ws, t[k], o[k]);
+                        t[k] = 0.f;
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < DPL; ++k) {
+        const size_t i = (size_t)item * HD + lane + 64 * k;
+        const float r = o[k] * inv;
+        if (out) out[i] = r;
+        if (out_hi) {
+            const __bf16 hb = (__bf16)r;
+            out_hi[i] = __builtin_bit_cast(uint16_t, hb);
+            out_lo[i] = __builtin_bit_cast(uint16_t, (__bf16)(r - (float)hb));
+        }
+    }
+}
+
+template <int HD, int G, bool FOLD>
+int launch_prefill_f32_blocks(const AttnArgs &a, int kv_heads, size_t rows, int S, int span, hipStream_t s) {
+    constexpr size_t lds = prefill_f32_lds_bytes<HD>();
+    constexpr int RB = 4 * (32 / G);  // rows of a block
+    static bool attr_set = false;
+    if (!attr_set) {
+        CHIP_CHECK(hipFuncSetAttribute((const void *)attn_prefill_f32_kernel<HD, G, FOLD>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        attr_set = true;
+    }
+    hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, G, FOLD>), dim3((unsigned)((rows + RB - 1) / RB), kv_heads, S),
+                       dim3(kThreads), lds, s, a, (int)rows, S, span, kF32PrefillSpan);
+    CHIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+// Prefill over an f32 cache: a row's keys are cut into parts of
+// kF32PrefillSpan keys, and into splits of j.span keys (a multiple); a split's
+// parts are folded in order, then the splits merged. Which blocks do it does
+// not change the bits: one block a split (its parts folded in registers), or
+// one a part (attn_merge_parts_kernel folds them), as many rows at a time as
+// the scratch holds the parts of. The second is for calls whose splits would
+// leave most of the chip idle while each block walks a long one: with splits
+// of 8,192 keys (a 64K cache), position 16,000, two Q4 layers with 32 q / 8 KV
+// heads of 128, 2 rows take 2,150 us a forward by split and 630 by part, 512
+// rows 3,120 and 4,090. The estimate: 7.5 us (3.2 at head_dim 64) for 64 keys
+// of a block and for a part's start; by split the longest block or all of them
+// over the CUs, by part rounds of blocks, a merge and its values' write and
+// read at 4.5 TB/s.
+template <int HD, int G>
+int launch_prefill_f32(const AttnJob &j, const AttnArgs &a, int S, hipStream_t s) {
+    constexpr size_t RB = 4 * (32 / G), sub = kF32PrefillSpan;
+    const int kvh = j.g.kv_heads;
+    if (j.span % sub || j.span <= (int)sub) {
+        CHIP_TRY((launch_prefill_f32_blocks<HD, G, false>(a, kvh, j.rows, S, j.span, s)));
+        return launch_merge2<HD>(j, a, S, s);
+    }
+    const size_t ctx = j.offset + j.rows, cus = (size_t)std::max(device_cus(), 1);
+    const size_t parts = (size_t)attention_prefill_splits(ctx, (int)sub);
+    const size_t row_floats = attention_part_floats(1, j.q_heads, (int)parts, HD);
+    const size_t fit = j.part ? std::min(j.part_floats / row_floats / RB * RB, (j.rows + RB - 1) / RB * RB) : 0;
+    if (parts > 1 && parts <= (size_t)kMaxParts && S <= 64 && fit > 0) {  // a wave of the merge holds a split per lane
+        constexpr float tile = HD == 64 ? 3.2f : 7.5f;
+        auto blocks = [&](size_t rows) { return (rows + RB - 1) / RB * (size_t)kvh; };  // of a split or part
+        const size_t launches = (j.rows + fit - 1) / fit, tiles = (ctx + 63) / 64;
+        const float by_split =
+            tile * (float)std::max(std::min(tiles, (size_t)j.span / 64), (blocks(j.rows) * tiles + cus - 1) / cus);
+        const float by_part =
+            (float)launches * (tile * (float)((blocks(fit) * parts + cus - 1) / cus * (sub / 64 + 1)) + 6.f) +
+            8.f * (float)(j.rows * row_floats) / 4.5e6f;
+        if (by_part < by_split) {
+            for (size_t r = 0; r < j.rows; r += fit) {
+                const size_t n = std::min(fit, j.rows - r), o = r * (size_t)j.q_heads * HD;
+                const int np = attention_prefill_splits(j.offset + r + n, (int)sub);
+                AttnArgs b = a;
+                b.q = a.q + r * j.q_stride;
+                b.offset = a.offset + (long)r;
+                if (b.out) b.out += o;
+                if (b.out_hi) b.out_hi += o, b.out_lo += o;
+                CHIP_TRY((launch_prefill_f32_blocks<HD, G, false>(b, kvh, n, np, (int)sub, s)));
+                if (np == 1) continue;  // one part: written as the output
+                const int items = (int)n * j.q_heads;
+                hipLaunchKernelGGL((attn_merge_parts_kernel<HD>), dim3((items + 3) / 4), dim3(kThreads), 0, s, b.part,
+                                   np, j.span / (int)sub, j.q_heads, items, b.out, b.out_hi, b.out_lo);
+                CHIP_CHECK(hipGetLastError());
+            }
+            return 0;
+        }
+    }
+    CHIP_TRY((launch_prefill_f32_blocks<HD, G, true>(a, kvh, j.rows, S, j.span, s)));
+    return launch_merge2<HD>(j, a, S, s);
+}
+
 template <int HD, int G>
 int launch_prefill_hg(const AttnJob &j, const AttnArgs &a, int S, hipStream_t s) {
+    if (j.g.kv_f32) return launch_prefill_f32<HD, G>(j, a, S, s);
     constexpr int RW = 32 / G;
+    constexpr size_t lds = (size_t)4 * 64 * HD * 2;
     const int rb = (int)((j.rows + 4 * RW - 1) / (4 * RW));
-    if (j.g.kv_f32) {
-        constexpr size_t lds = prefill_f32_lds_bytes<HD>();
-        static bool attr_set = false;
-        if (!attr_set) {
-            CHIP_CHECK(hipFuncSetAttribute((const void *)attn_prefill_f32_kernel<HD, G>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            attr_set = true;
-        }
-        hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, G>), dim3(rb, j.g.kv_heads, S), dim3(kThreads), lds, s, a,
-                           (int)j.rows, S, j.span);
-    } else {
-        constexpr size_t lds = (size_t)4 * 64 * HD * 2;
-        static bool attr_set = false;
-        if (!attr_set) {
-            CHIP_CHECK(hipFuncSetAttribute((const void *)attn_prefill_kernel<HD, G>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            attr_set = true;
-        }
-        hipLaunchKernelGGL((attn_prefill_kernel<HD, G>), dim3(rb, j.g.kv_heads, S), dim3(kThreads), lds, s, a,
-                           (int)j.rows, S, j.span);
+    static bool attr_set = false;
+    if (!attr_set) {
+        CHIP_CHECK(hipFuncSetAttribute((const void *)attn_prefill_kernel<HD, G>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        attr_set = true;
     }
+    hipLaunchKernelGGL((attn_prefill_kernel<HD, G>), dim3(rb, j.g.kv_heads, S), dim3(kThreads), lds, s, a, (int)j.rows,
+                       S, j.span);
     CHIP_CHECK(hipGetLastError());
-    if (S > 1) {
-        const int items = (int)j.rows * j.q_heads;
-        hipLaunchKernelGGL((attn_merge2_kernel<HD>), dim3((items + 3) / 4), dim3(kThreads), 0, s, a.part, S,
-                           j.q_heads, items, a.out, a.out_hi, a.out_lo);
-        CHIP_CHECK(hipGetLastError());
-    }
-    return 0;
+    return launch_merge2<HD>(j, a, S, s);
 }
 
 template <int HD>
@@ -1476,7 +1663,8 @@ int attention_prefill_splits(size_t ctx, int span) {
 // on 512-row chunks at up to 8K keys (Llama-3-8B) 20,766 tok/s with 1,024,
 // 19,178 with 4,096. Capacity / 8 picks 4,096 for the 33K cache and 1,024
 // for the 8K one. The f32 kernel runs one block per CU and a tile takes it
-// about three times as long, so short caches take spans from 256 on.
+// about three times as long, so short caches take spans from 256 on (longer
+// ones run part by part where that is faster, launch_prefill_f32).
 int attention_prefill_span(size_t kv_capacity, bool kv_f32) {
     int span = kv_f32 ? kF32PrefillSpan : kDefaultPrefillSpan;
     while ((size_t)span * 2 <= kv_capacity / 8 && span < (1 << 20)) span *= 2;

@@ -167,7 +167,7 @@ int launch_gather_rows(const uint8_t *src, uint8_t *dst, const int32_t *map, siz
 // Keys per split of the matrix-core chunked prefill when the caller names
 // no span (attention_prefill_span gives a model's).
 constexpr int kDefaultPrefillSpan = 1024;
-// Shortest span over an f32 cache.
+// Shortest span over an f32 cache; longer ones are folded from parts of it.
 constexpr int kF32PrefillSpan = 256;
 
 struct AttnJob {

@@ -142,6 +142,27 @@ def test_f32_kv_prefill_attention_tile_and_span_edges(hip, oracle, shape):
         assert rel_err(got, ref) < 5e-5, (n, chunk)
 
 
+@pytest.mark.parametrize("shape", TINY, ids=lambda s: s.name)
+def test_f32_kv_long_cache_bits_independent_of_chunks(hip, shape):
+    """An f32 cache of 16,384 positions attends in splits of 2,048 keys, folded
+    from parts of 256 in registers (chunks of 160 rows, whose parts the scratch
+    does not hold) or by the merge (few rows): every position's K and V of the
+    second layer and the last logits are the same bits either way, at the edges
+    of parts and splits."""
+    toks = synth.make_tokens(shape.vocab_size, 4200, seed=31)
+    g = hip.HipForward(shape, weights(shape), kv="f32", kv_capacity=16384, max_chunk_rows=160)
+    cuts = (0, 200, 255, 259, 510, 515, 2040, 2047, 2052, 2300, 4090, 4097, 4099, 4104, 4200)
+    want = g.forward(toks, 0, chunk_rows=160)
+    k0, v0 = g.kv_rows(1, 0, len(toks))
+    g.clear_cache()
+    for a, b in zip(cuts, cuts[1:]):
+        got = g.forward(toks[a:b], a, chunk_rows=160 if b - a > 100 else 7)
+    k1, v1 = g.kv_rows(1, 0, len(toks))
+    assert np.array_equal(bits(k0), bits(k1)) and np.array_equal(bits(v0), bits(v1))
+    assert np.array_equal(bits(got), bits(want))
+    assert np.isfinite(want).all() and np.abs(k0).max() > 0
+
+
 @pytest.mark.parametrize("kv", ["bf16", "f32"])
 def test_kv_continuation_bit_exact_on_device(hip, kv):
     # decoder.rs:1710-1728: prefill in one call == prefill in two calls.
