@@ -1346,24 +1346,28 @@ __global__ __launch_bounds__(kThreads) void attn_merge2_kernel(const float *part
     static_assert(kMaxSplits <= 128, "a lane holds two splits");
     const int s1 = lane + 64;
     const float m0 = lane < S ? p[(size_t)lane * (HD + 2) + HD] : -INFINITY;
-    const float m1 = s1 < S ? p[(size_t)s1 * (HD + 2) + HD] : -INFINITY;
+    float m1 = -INFINITY, w1 = 0.f;
+    if (S > 64 && s1 < S) m1 = p[(size_t)s1 * (HD + 2) + HD];
     const float M = wave_max(fmaxf(m0, m1));
     const float w0 = m0 == -INFINITY ? 0.f : exp2f(m0 - M);
-    const float w1 = m1 == -INFINITY ? 0.f : exp2f(m1 - M);
-    const float L = wave_sum(w0 != 0.f ? w0 * p[(size_t)lane * (HD + 2) + HD + 1] : 0.f) +
-                    wave_sum(w1 != 0.f ? w1 * p[(size_t)s1 * (HD + 2) + HD + 1] : 0.f);
+    float L = wave_sum(w0 != 0.f ? w0 * p[(size_t)lane * (HD + 2) + HD + 1] : 0.f);
+    if (S > 64) {
+        w1 = m1 == -INFINITY ? 0.f : exp2f(m1 - M);
+        L += wave_sum(w1 != 0.f ? w1 * p[(size_t)s1 * (HD + 2) + HD + 1] : 0.f);
+    }
     const float inv = 1.0f / L;
     constexpr int DPL = HD / 64;  // dims per lane
     float o[DPL];
 #pragma unroll
     for (int k = 0; k < DPL; ++k) o[k] = 0.f;
-    for (int s = 0; s < S; ++s) {
-        const float ws = s < 64 ? __shfl(w0, s, 64) : __shfl(w1, s - 64, 64);
+    auto fold = [&](float ws, int s) {
         if (ws != 0.f) {
 #pragma unroll
             for (int k = 0; k < DPL; ++k) o[k] = fmaf(ws, p[(size_t)s * (HD + 2) + lane + 64 * k], o[k]);
         }
-    }
+    };
+    for (int s = 0; s < min(S, 64); ++s) fold(__shfl(w0, s, 64), s);
+    for (int s = 64; s < S; ++s) fold(__shfl(w1, s - 64, 64), s);
 #pragma unroll
     for (int k = 0; k < DPL; ++k) {
         const size_t i = (size_t)item * HD + lane + 64 * k;
