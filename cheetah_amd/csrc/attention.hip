@@ -1061,6 +1061,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 // 128: 40 / 80 / 128 us a chunk against 1,025 to 1,781 us on the vector ALUs
 // (attn_kernel, which decodes only now); that prompt through two Q4 layers of
 // the shape 11.94 -> 4.36 ms, its logits no further from 64-bit ones.
+//
+// Infinities and NaN as f32 products give them (plain_row): the parts do not
+// carry them. Staging clamps V, the scores' NaN shows in the weight sum; 0.4 %
+// of that prompt's time, 2 to 3 % of a 512-row chunk's deep in a long cache.
 // ---------------------------------------------------------------------------
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 
@@ -1094,7 +1098,7 @@ __device__ __forceinline__ void split3x8(const float (&v)[8], bf16x8 (&out)[3]) 
 
 constexpr int kF32LdV = 64 + 8;  // transposed V row: 64 positions + 16 bytes
 template <int HD>
-constexpr size_t prefill_f32_lds_bytes() { return (size_t)3 * 2 * (64 * HD + HD * kF32LdV); }
+constexpr size_t prefill_f32_lds_bytes() { return (size_t)3 * 2 * (64 * HD + HD * kF32LdV) + 16; }
 
 // One more part of a row's softmax (maximum m, weight sum l, values o) folded
 // into the running one (M, L, O), parts in order; a part without a key (m =
@@ -1108,6 +1112,71 @@ __device__ __forceinline__ void fold_factors(float m, float &M, float &alpha, fl
 }
 __device__ __forceinline__ float fold_value(float O, float o, float alpha, float beta) {
     return fmaf(beta, o, O * alpha);
+}
+
+// 2^119: weights of up to 2^8 take the product with a larger V past the largest
+// number.
+constexpr float kBigV = 0x1p119f;
+
+// One row's attention over positions [p0, p1) in plain f32 products, parts of
+// `sub` positions folded in order, a lane's HD / 2 dims of it stored as
+// store_prefill_rows does: the rare rows whose operands the BF16 parts do not
+// carry. A call, so that it takes no registers of the loop's.
+template <int HD>
+__device__ __attribute__((noinline)) void plain_row(AttnArgs a, int row, int head, int g, int half, int p0, int p1, int sub,
+                                              float *part, int S) {
+    constexpr int UT = HD / 32;
+    const float *qp = a.q + (size_t)row * a.q_stride + (size_t)head * HD;
+    const float sl2 = (1.0f / sqrtf((float)HD)) * 1.44269504088896340736f;
+    f32x16 o[UT];
+    float M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int u = 0; u < UT; ++u) o[u] = f32x16{};
+#pragma unroll 1
+    for (; p0 < p1; p0 += sub) {
+        f32x16 t[UT];
+        float m = -INFINITY, l = 0.f;
+#pragma unroll
+        for (int u = 0; u < UT; ++u) t[u] = f32x16{};
+#pragma unroll 1
+        for (int p = p0; p < min(p0 + sub, p1); ++p) {
+            const size_t at = (((size_t)a.page_table[p / a.page_size] * a.kv_heads + g) * a.page_size + p % a.page_size) * HD;
+            const float *kp = (const float *)a.k + at, *vp = (const float *)a.v + at + 4 * half;
+            float dot = 0.f;
+#pragma unroll 1
+            for (int d = 0; d < HD; d += 16) {
+                f32x4 q[4], k[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) q[i] = *(const f32x4 *)(qp + d + 4 * i), k[i] = *(const f32x4 *)(kp + d + 4 * i);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) dot = fmaf(k[i][e], q[i][e], dot);
+            }
+            const float s = dot * sl2, mn = fmaxf(m, s);
+            const float alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+            const float w = s == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s - mn);
+            m = mn;
+            l = l * alpha + w;
+#pragma unroll
+            for (int u = 0; u < UT; ++u)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const f32x4 v = *(const f32x4 *)(vp + 32 * u + 8 * q);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) t[u][4 * q + e] = fmaf(w, v[e], t[u][4 * q + e] * alpha);
+                }
+        }
+        float alpha, beta;
+        const bool any = m != -INFINITY;
+        fold_factors(m, M, alpha, beta);
+        L = any ? fold_value(L, l, alpha, beta) : L;
+#pragma unroll
+        for (int u = 0; u < UT; ++u)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[u][r] = any ? fold_value(o[u][r], t[u][r], alpha, beta) : o[u][r];
+    }
+    store_prefill_rows<HD>(a, o, M, L, part, (size_t)row * a.q_heads * HD + (size_t)head * HD, S, half);
 }
 
 // FOLD: the block's split is longer than `sub` keys; its parts of `sub` keys
@@ -1124,6 +1193,7 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
     extern __shared__ __attribute__((aligned(16))) uint16_t smem_f32[];
     uint16_t *ks = smem_f32;               // [3][64][HD], chunks swizzled as in attn_prefill_kernel
     uint16_t *vt = smem_f32 + 3 * 64 * HD;  // [3][HD][LDV]
+    int *big_pos = (int *)(vt + 3 * HD * LDV);  // first position with a V value of kBigV or more
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = lane & 31, half = lane >> 5;
     const int rb = blockIdx.x, g = blockIdx.y, split = blockIdx.z;
@@ -1167,7 +1237,19 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
                                              : f32x4{0.f, 0.f, 0.f, 0.f};
         }
     };
+    // V values of kBigV or more (infinities; NaN comes out as -kBigV) are staged
+    // as +-kBigV: as 0 x V they reach no row that does not see them.
+    float top = 0.f;
     auto stage = [&]() {
+#pragma unroll
+        for (int c = 0; c < VU; ++c)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    vr[c][i][e] = __builtin_amdgcn_fmed3f(vr[c][i][e], -kBigV, kBigV);
+                    top = fmaxf(top, fabsf(vr[c][i][e]));
+                }
 #pragma unroll
         for (int c = 0; c < KU; ++c) {
             const int idx = tid + kThreads * c, r = krow_of(idx / CPR);
@@ -1192,9 +1274,9 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
             }
         }
     };
-    fetch(start, page_of(start));
     const int last_tile = start + (end - 1 - start) / 64 * 64;
-    int page_next = page_of(min(start + 64, last_tile));
+    fetch(start, page_of(start));
+    if (tid == 0) *big_pos = INT32_MAX;
 
     // Q^T operands, pre-scaled by log2(e) / sqrt(HD) (scores in the exp2 domain).
     bf16x8 q3[KSTEPS][3];
@@ -1216,14 +1298,16 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
         }
     }
 
-    f32x16 oacc[UT];
+    f32x16 oacc[UT], osum[FOLD ? UT : 1];
+    float m2, l, msum = -INFINITY, lsum = 0.f;
+    bool odd = false;  // a score of the row's is NaN
 #pragma unroll
     for (int u = 0; u < UT; ++u) oacc[u] = f32x16{};
-    float m2 = -INFINITY, l = 0.f;
-    f32x16 osum[FOLD ? UT : 1];
 #pragma unroll
     for (int u = 0; u < (FOLD ? UT : 1); ++u) osum[u] = f32x16{};
-    float msum = -INFINITY, lsum = 0.f;
+    m2 = msum = -INFINITY;
+    l = lsum = 0.f;
+    int page_next = page_of(min(start + 64, last_tile));
     for (int t0 = start; t0 < end; t0 += 64) {
         __syncthreads();  // the previous tile's reads are done
         stage();
@@ -1265,7 +1349,7 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
             const bool raise = tmax > m2 + 8.0f;
             if (__any(raise)) {
                 const float mnew = raise ? tmax : m2;
-                const float alpha = __builtin_amdgcn_exp2f(m2 - mnew);  // 1 where not raised, 0 from -inf
+                const float alpha = raise ? __builtin_amdgcn_exp2f(m2 - mnew) : 1.f;  // 0 from -inf
                 l *= alpha;
 #pragma unroll
                 for (int u = 0; u < UT; ++u)
@@ -1310,6 +1394,7 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
                 // A part without a key of the row may hold NaN (its -inf maximum
                 // rescaled with its neighbours'): left out, as the merge does.
                 const bool any = m2 != -INFINITY;
+                odd |= l != l && my_pos >= t0 / sub * sub;
                 float alpha, beta;
                 fold_factors(m2, msum, alpha, beta);
                 lsum = any ? fold_value(lsum, l, alpha, beta) : lsum;
@@ -1324,6 +1409,25 @@ __global__ __launch_bounds__(kThreads, HD == 64 ? 2 : 1) void attn_prefill_f32_k
                 l = 0.f;
             }
         }
+    }
+    // The parts of an infinite operand, or of a product past the largest
+    // number, add up to NaN where the f32 product is an infinity (a score of
+    // -inf weighs nothing). The rows with a NaN score, or with a V value of kBigV
+    // or more in sight, are computed again in plain f32, over their own keys.
+    if constexpr (!FOLD) odd = l != l;
+    odd = odd && my_pos >= start;
+    if (__syncthreads_or(top >= kBigV)) {
+        for (int e = tid; e < (end - start) * HD; e += kThreads) {
+            const int p = start + e / HD;
+            const float v = vbase[(((size_t)page_of(p) * a.kv_heads + g) * a.page_size + p % a.page_size) * HD + e % HD];
+            if (!(fabsf(v) < kBigV)) atomicMin(big_pos, p);
+        }
+        __syncthreads();
+        odd = odd || *big_pos <= my_pos;
+    }
+    if (rvalid && odd) {
+        plain_row<HD>(a, row, head, g, half, start, min(end, my_pos + 1), FOLD ? sub : span, part, S);
+        return;
     }
     if (!rvalid) return;
     const size_t ob = (size_t)row * a.q_heads * HD + (size_t)head * HD;
@@ -1504,15 +1608,15 @@ template <int HD, int G>
 int launch_prefill_f32(const AttnJob &j, const AttnArgs &a, int S, hipStream_t s) {
     constexpr size_t RB = 4 * (32 / G), sub = kF32PrefillSpan;
     const int kvh = j.g.kv_heads;
-    if (j.span % sub || j.span <= (int)sub) {
+    const size_t ctx = j.offset + j.rows, cus = (size_t)std::max(device_cus(), 1);
+    const size_t parts = (size_t)attention_prefill_splits(ctx, (int)sub);
+    if (j.span % sub || j.span <= (int)sub || parts == 1) {  // nothing to fold
         CHIP_TRY((launch_prefill_f32_blocks<HD, G, false>(a, kvh, j.rows, S, j.span, s)));
         return launch_merge2<HD>(j, a, S, s);
     }
-    const size_t ctx = j.offset + j.rows, cus = (size_t)std::max(device_cus(), 1);
-    const size_t parts = (size_t)attention_prefill_splits(ctx, (int)sub);
     const size_t row_floats = attention_part_floats(1, j.q_heads, (int)parts, HD);
     const size_t fit = j.part ? std::min(j.part_floats / row_floats / RB * RB, (j.rows + RB - 1) / RB * RB) : 0;
-    if (parts > 1 && parts <= (size_t)kMaxParts && S <= 64 && fit > 0) {  // a wave of the merge holds a split per lane
+    if (parts <= (size_t)kMaxParts && S <= 64 && fit > 0) {  // a wave of the merge holds a split per lane
         constexpr float tile = HD == 64 ? 3.2f : 7.5f;
         auto blocks = [&](size_t rows) { return (rows + RB - 1) / RB * (size_t)kvh; };  // of a split or part
         const size_t launches = (j.rows + fit - 1) / fit, tiles = (ctx + 63) / 64;

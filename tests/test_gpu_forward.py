@@ -163,6 +163,76 @@ def test_f32_kv_long_cache_bits_independent_of_chunks(hip, shape):
     assert np.isfinite(want).all() and np.abs(k0).max() > 0
 
 
+def _marked_model(head_dim, edit):
+    """A two-layer qwen2 shape whose token 7 alone has a value at hidden unit 5
+    (so a weight column 5 speaks of it alone), its units changed by
+    `edit(units, shape)`: BF16 arrays by unit id."""
+    shape = configs.TINY_QWEN2.replace(name=f"marked-{head_dim}", head_dim=head_dim)
+    w = {k: synth.bf16_to_f32(v).copy() for k, v in synth.make_weights(shape).items()}
+    w["model.embed_tokens.weight"][:, 5] = 0.0
+    w["model.embed_tokens.weight"][7, 5] = 1.0
+    edit(w, shape)
+    return shape, {k: synth.f32_to_bf16(v) for k, v in w.items()}
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("capacity", [640, 16384])
+def test_f32_kv_infinite_value_reaches_no_earlier_row(hip, head_dim, capacity):
+    """Layer 0 gives token 7 infinite V values: the rows before it, in the same
+    tile of the same call, keep the bits that a call without it gives them;
+    the rows after it see the infinities."""
+    def edit(w, shape):
+        w["model.layers.0.self_attn.v_proj.weight"][3::64, 5] = 3e38
+
+    shape, w = _marked_model(head_dim, edit)
+    g = hip.HipForward(shape, w, kv="f32", kv_capacity=capacity, max_chunk_rows=160)
+    toks = synth.make_tokens(shape.vocab_size, 300, seed=12)
+    toks[toks == 7] = 8
+    for at in (3, 70, 290):
+        g.clear_cache()
+        g.forward(toks[:at], 0, chunk_rows=160)
+        want = g.kv_rows(1, 0, at)
+        g.clear_cache()
+        both = toks.copy()
+        both[at] = 7
+        assert not np.isfinite(g.forward(both, 0, chunk_rows=160)).all()
+        assert np.isinf(g.kv_rows(0, at, 1)[1]).any()
+        got = g.kv_rows(1, 0, at)
+        for x, y in zip(got, want):
+            assert np.isfinite(y).all()
+            assert np.array_equal(bits(x), bits(y)), at
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("capacity", [640, 16384])
+def test_f32_kv_score_of_minus_infinity_weighs_nothing(hip, oracle, head_dim, capacity):
+    """Token 7's keys and every query hold large values of opposite signs in the
+    slowest rotary pair: their product is past the largest f32, -inf, and
+    weighs nothing. The logits are finite and the oracle's within 5e-5 (the
+    GEMMs' hi/lo input split, as in the tile and span edges test)."""
+    def edit(w, shape):
+        hd = shape.head_dim
+        p = "model.layers.0.self_attn."
+        w[p + "k_proj.weight"][hd // 2 - 1::hd, 5] = 1e29
+        w[p + "q_proj.weight"][hd // 2 - 1::hd] = 0.0
+        w[p + "q_proj.weight"][hd // 2 - 1::hd, 6:] = 1e13 * np.sign(w[p + "q_proj.weight"][:1, 6:] + 1e-6)
+        w[p + "q_proj.bias"][hd // 2 - 1::hd] = -1e15
+
+    shape, w = _marked_model(head_dim, edit)
+    g = hip.HipForward(shape, w, kv="f32", kv_capacity=capacity, max_chunk_rows=160)
+    r = oracle.RefModel(shape, w)
+    toks = synth.make_tokens(shape.vocab_size, 300, seed=13)
+    toks[toks == 7] = 8
+    toks[[1, 40, 280]] = 7
+    for n in (4, 60, 300):
+        g.clear_cache()
+        r.clear_cache()
+        got = g.forward(toks[:n], 0, chunk_rows=160)
+        ref = r.forward(toks[:n], 0, chunk_rows=256)
+        assert np.isfinite(ref).all()
+        assert rel_err(got, ref) < 5e-5, n
+
+
 @pytest.mark.parametrize("kv", ["bf16", "f32"])
 def test_kv_continuation_bit_exact_on_device(hip, kv):
     # decoder.rs:1710-1728: prefill in one call == prefill in two calls.
