@@ -40,6 +40,14 @@ void set_error(const std::string &message) { g_error = message; }
 const char *last_error() { return g_error.c_str(); }
 hipStream_t lib_stream() { return g_stream; }
 
+int allow_dynamic_lds(const void *fn, size_t bytes, std::atomic<uint64_t> &done) {
+    const uint64_t bit = 1ull << g_device;  // below kMaxDevices once initialized
+    if (done.load(std::memory_order_acquire) & bit) return 0;
+    CHIP_CHECK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    done.fetch_or(bit, std::memory_order_release);
+    return 0;
+}
+
 int ensure_ready() {
     if (!g_ready) return fail("HIP backend: not initialized; call cheetah_hip_init first.");
     CHIP_CHECK(hipSetDevice(g_device));

@@ -1579,12 +1579,8 @@ template <int HD, int G, bool FOLD>
 int launch_prefill_f32_blocks(const AttnArgs &a, int kv_heads, size_t rows, int S, int span, hipStream_t s) {
     constexpr size_t lds = prefill_f32_lds_bytes<HD>();
     constexpr int RB = 4 * (32 / G);  // rows of a block
-    static bool attr_set = false;
-    if (!attr_set) {
-        CHIP_CHECK(hipFuncSetAttribute((const void *)attn_prefill_f32_kernel<HD, G, FOLD>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr_set = true;
-    }
+    static std::atomic<uint64_t> lds_set{0};
+    CHIP_TRY(allow_dynamic_lds((const void *)attn_prefill_f32_kernel<HD, G, FOLD>, lds, lds_set));
     hipLaunchKernelGGL((attn_prefill_f32_kernel<HD, G, FOLD>), dim3((unsigned)((rows + RB - 1) / RB), kv_heads, S),
                        dim3(kThreads), lds, s, a, (int)rows, S, span, kF32PrefillSpan);
     CHIP_CHECK(hipGetLastError());
@@ -1654,12 +1650,8 @@ int launch_prefill_hg(const AttnJob &j, const AttnArgs &a, int S, hipStream_t s)
     constexpr int RW = 32 / G;
     constexpr size_t lds = (size_t)4 * 64 * HD * 2;
     const int rb = (int)((j.rows + 4 * RW - 1) / (4 * RW));
-    static bool attr_set = false;
-    if (!attr_set) {
-        CHIP_CHECK(hipFuncSetAttribute((const void *)attn_prefill_kernel<HD, G>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr_set = true;
-    }
+    static std::atomic<uint64_t> lds_set{0};
+    CHIP_TRY(allow_dynamic_lds((const void *)attn_prefill_kernel<HD, G>, lds, lds_set));
     hipLaunchKernelGGL((attn_prefill_kernel<HD, G>), dim3(rb, j.g.kv_heads, S), dim3(kThreads), lds, s, a, (int)j.rows,
                        S, j.span);
     CHIP_CHECK(hipGetLastError());

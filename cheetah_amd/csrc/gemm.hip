@@ -816,12 +816,8 @@ int launch_ring(GArgs a, int split, hipStream_t s) {
     constexpr int BM = 32 * MT * WM, BNO = (DUAL ? 32 : 64) * WN;
     if (!a.n_tiles) a.n_tiles = (a.N - a.n_first + BNO - 1) / BNO;
     constexpr size_t lds = ring_lds_bytes<FMT, MT, WM, WN, NS>();
-    static bool attr_set = false;
-    if (!attr_set) {
-        CHIP_CHECK(hipFuncSetAttribute((const void *)gemm_ring_kernel<FMT, DUAL, MT, WM, WN, NS, QG>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        attr_set = true;
-    }
+    static std::atomic<uint64_t> lds_set{0};
+    CHIP_TRY(allow_dynamic_lds((const void *)gemm_ring_kernel<FMT, DUAL, MT, WM, WN, NS, QG>, lds, lds_set));
     const dim3 grid(a.n_tiles * ((a.M + BM - 1) / BM), 1, split ? a.nstored : 1);
     hipLaunchKernelGGL((gemm_ring_kernel<FMT, DUAL, MT, WM, WN, NS, QG>), grid, dim3(64 * WM * WN), lds, s, a, split);
     CHIP_CHECK(hipGetLastError());

@@ -2,6 +2,8 @@
 // shapes it is given before touching the device and returns 0 / -1.
 #pragma once
 
+#include <atomic>
+
 #include "common.hpp"
 
 namespace chip {
@@ -10,6 +12,11 @@ namespace chip {
 size_t device_max_lds();
 int device_cus();
 size_t device_lds_per_cu();
+
+// Lets kernel `fn` take `bytes` of dynamic LDS on the library's device. `done`
+// is the caller's static for this kernel, a bit per device: set once on each,
+// from any thread.
+int allow_dynamic_lds(const void *fn, size_t bytes, std::atomic<uint64_t> &done);
 
 // ---------------------------------------------------------------------------
 // Weight matrix in device memory, in the reference's layout.

@@ -268,6 +268,30 @@ def test_attention_prefill_merges_more_than_64_splits(hip, hd, ctx):
         assert rel_err(got[row], ref) < 2e-5, row
 
 
+def test_attention_prefill_first_calls_from_several_threads(hip, oracle):
+    """The first call of a kernel lets it take its LDS, from whichever thread
+    comes first: eight threads at once, each with its own buffers and scratch."""
+    import threading
+
+    rng = np.random.default_rng(11)
+    k, v, q = _attn_case(rng, 15, 5, 128, 70, 6)
+    kp, vp, table = hip.paged_kv(k, v, seed=2)
+    got = [None] * 8
+
+    def run(i):
+        got[i] = hip.attention(q, kp, vp, table, 15, 6, 64)
+
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(8)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    kf, vf = synth.bf16_to_f32(k), synth.bf16_to_f32(v)
+    ref = np.stack([oracle.attention(kf, vf, q[r], 15, 5, 128, 64 + r) for r in range(6)])
+    for g in got:
+        assert np.max(np.abs(g - ref)) < 1e-4
+
+
 @pytest.mark.parametrize("q_heads,kv_heads,hd,offset,rows", [(14, 2, 64, 0, 37), (32, 8, 128, 100, 70),
                                                             (28, 4, 128, 4000, 9)])
 def test_attention_prefill_rows_match_oracle(hip, oracle, q_heads, kv_heads, hd, offset, rows):
