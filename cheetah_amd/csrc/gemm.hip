@@ -1090,9 +1090,10 @@ int launch_split_bf16_rows(const float *x, size_t n, size_t cols, size_t stride,
                            hipStream_t s) {
     if (stride == cols) return launch_split_bf16(x, n * cols, xh, xl, s);
     if (n == 0) return 0;
-    if (!x || !xh || !xl || stride < cols || stride % 4 || stride > (size_t)INT32_MAX || ((uintptr_t)xh % 8) ||
-        ((uintptr_t)xl % 8))
-        return fail("HIP backend: split needs rows padded to a multiple of 4 and 8-byte aligned halves.");
+    if (!x || !xh || !xl || stride < cols || stride % 4 || stride > (size_t)INT32_MAX || ((uintptr_t)x % 16) ||
+        ((uintptr_t)xh % 8) || ((uintptr_t)xl % 8))
+        return fail("HIP backend: split needs 16-byte aligned input, rows padded to a multiple of 4 and 8-byte aligned "
+                    "halves.");
     const size_t blocks = (n * stride / 4 + kThreads - 1) / kThreads;
     if (blocks > (size_t)INT32_MAX) return fail("HIP backend: split shape too large.");
     hipLaunchKernelGGL(split_bf16_rows_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, s, x, n, (int)cols,

@@ -221,6 +221,23 @@ def _attn_case(rng, q_heads, kv_heads, hd, ctx, rows):
     return k, v, q
 
 
+@pytest.mark.parametrize("fmt", ["bf16", "q8", "q4"])
+@pytest.mark.parametrize("cols", [32, 33, 40])
+def test_gemm_refuses_an_input_off_16_bytes(hip, fmt, cols):
+    """Every format and column count, padded to whole stages or not."""
+    rng = np.random.default_rng(cols)
+    rows, n = 8, 3
+    w = rng.integers(0, 16000, (rows, cols)).astype(np.uint16) if fmt == "bf16" else random_quant(rng, fmt, rows, cols)
+    wd = hip.DeviceBuffer.from_array(w)
+    xd = hip.DeviceBuffer.from_array(np.zeros(n * cols + 4, np.float32))
+    yd = hip.DeviceBuffer(n * rows * 4)
+    fn = getattr(hip.lib(), f"cheetah_hip_gemm_{fmt}")
+    for off in (4, 8, 12):
+        with pytest.raises(hip.HipError, match="aligned"):
+            hip.check(fn(wd.ptr, rows, cols, xd.ptr + off, n, yd.ptr))
+    hip.check(fn(wd.ptr, rows, cols, xd.ptr + 16, n, yd.ptr))
+
+
 @pytest.mark.parametrize("q_heads,kv_heads,hd", [(14, 2, 64), (32, 8, 128), (28, 4, 128), (4, 4, 64), (8, 1, 64)])
 @pytest.mark.parametrize("ctx", [1, 63, 64, 65, 1000, 4096])
 def test_attention_decode_matches_oracle(hip, oracle, q_heads, kv_heads, hd, ctx):
