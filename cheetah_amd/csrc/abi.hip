@@ -389,8 +389,8 @@ int cheetah_hip_time_gemv(uint32_t fmt, const void *const *w, size_t nbuf, size_
 int cheetah_hip_time_gemm(uint32_t fmt, const void *const *w, size_t nbuf, size_t rows, size_t cols,
                           const float *x, size_t n, float *y, size_t iters, float *ms) {
     CHIP_TRY(ensure_ready());
-    if (!w || nbuf == 0 || iters == 0 || !ms || !x || !y || n == 0)
-        return fail("HIP backend: time_gemm needs buffers, rows and iterations.");
+    if (!w || nbuf == 0 || iters == 0 || !ms || !x || !y || n == 0 || rows == 0 || cols == 0)
+        return fail("HIP backend: time_gemm needs buffers, rows, columns and iterations.");
     if (fmt != FMT_BF16 && fmt != FMT_Q8 && fmt != FMT_Q4) return fail("HIP backend: unknown weight format.");
     for (size_t i = 0; i < nbuf; ++i)
         if (!w[i]) return fail("HIP backend: time_gemm with a null weight buffer.");

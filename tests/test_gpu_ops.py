@@ -238,6 +238,18 @@ def test_gemm_refuses_an_input_off_16_bytes(hip, fmt, cols):
     hip.check(fn(wd.ptr, rows, cols, xd.ptr + 16, n, yd.ptr))
 
 
+@pytest.mark.parametrize("rows,cols", [(0, 64), (64, 0)])
+def test_time_gemm_refuses_an_empty_matrix(hip, rows, cols):
+    """Before its workspace is planned (a division by the column count)."""
+    import ctypes
+
+    buf = hip.DeviceBuffer(4096)
+    ms = ctypes.c_float(0)
+    with pytest.raises(hip.HipError, match="columns"):
+        hip.check(hip.lib().cheetah_hip_time_gemm(1, (ctypes.c_void_p * 1)(buf.ptr), 1, rows, cols, buf.ptr, 4, buf.ptr,
+                                                  1, ctypes.byref(ms)))
+
+
 @pytest.mark.parametrize("q_heads,kv_heads,hd", [(14, 2, 64), (32, 8, 128), (28, 4, 128), (4, 4, 64), (8, 1, 64)])
 @pytest.mark.parametrize("ctx", [1, 63, 64, 65, 1000, 4096])
 def test_attention_decode_matches_oracle(hip, oracle, q_heads, kv_heads, hd, ctx):
