@@ -665,11 +665,13 @@ int init_instance(cheetah_hip_model *m) {
     }
     m->epoch = sh.epoch;
     CHIP_TRY(m->mem.alloc(&m->hidden, R * H));
-    CHIP_TRY(m->mem.alloc(&m->normed, R * H));
     CHIP_TRY(m->mem.alloc(&m->qkv, R * (qd + 2 * kvd)));
-    CHIP_TRY(m->mem.alloc(&m->attn, R * qd));
     CHIP_TRY(m->mem.alloc(&m->qrot, R * qd));
-    CHIP_TRY(m->mem.alloc(&m->act, R * c.intermediate_size));
+    // f32 GEMM inputs: a chunk's only where the width rules the halves out
+    // (enqueue_chunk), a decode step's one row of attention and activations.
+    if (!gemm_takes_halves(H)) CHIP_TRY(m->mem.alloc(&m->normed, R * H));
+    CHIP_TRY(m->mem.alloc(&m->attn, (gemm_takes_halves(qd) ? 1 : R) * qd));
+    CHIP_TRY(m->mem.alloc(&m->act, (gemm_takes_halves(c.intermediate_size) ? 1 : R) * c.intermediate_size));
     CHIP_TRY(m->mem.alloc(&m->logits, c.vocab_size));
     // Prefill partials: the span splits at full capacity; decode:
     // attention_max_splits.

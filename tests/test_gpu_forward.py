@@ -249,6 +249,36 @@ def test_kv_continuation_bit_exact_on_device(hip, kv):
         assert np.array_equal(bits(g.forward(toks[i:i + 1], i)), bits(dec_full[i - 70])), i
 
 
+def test_chunk_buffers_hold_what_a_chunk_reads(hip):
+    """Device memory of 8,192 more chunk rows: the hidden, qkv and rotated query
+    rows, the BF16 halves and the attention partials, and no f32 copies of the
+    GEMMs' inputs (1 KiB + 32 KiB a row here). 100 MiB for split sums."""
+    import ctypes
+
+    runtime = ctypes.CDLL("libamdhip64.so.7")  # the one that the library runs on
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert runtime.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    shape = configs.TINY_QWEN2.replace(name="wide", intermediate_size=8192)
+    units = synth.make_weights(shape)
+
+    def used(rows):
+        before = free_bytes()
+        g = hip.HipForward(shape, units, kv_capacity=512, max_chunk_rows=rows)
+        taken = before - free_bytes()
+        g.close()
+        return taken
+
+    used(64)  # the library's first model: code and queues
+    more = used(9216) - used(1024)
+    inter, hidden, qd, kvd = shape.intermediate_size, shape.hidden_size, shape.q_dim, shape.kv_dim
+    row = 4 * (hidden + 2 * qd + 2 * kvd) + 2 * 4 * inter + 4 * shape.q_heads * (shape.head_dim + 2)
+    assert 8192 * row <= more < 8192 * row + (100 << 20), more / 8192
+
+
 def test_snapshot_restore_clone_bit_exact_on_device(hip):
     # decoder.rs:1761-1818: a clone starts empty; snapshot -> restore ->
     # continue equals the uninterrupted run, including a restore that ends
