@@ -124,6 +124,104 @@ def test_mixed_forward_calls_agree_with_device_greedy(hip, shape, quant):
     assert got == want
 
 
+@pytest.mark.parametrize("quant", [None, "q4"])
+@pytest.mark.parametrize("shape", TINY, ids=lambda s: s.name)
+def test_decode_logits_are_the_same_bits_with_and_without_sampling(hip, shape, quant):
+    """One decode position on one restored cache through forward (no argmax) and
+    forward_greedy, on the persistent kernel and the decode graphs, another
+    token between them: all logits bit for bit, and the last ones (an odd
+    vocabulary ends inside a vector store) not the other token's."""
+    from cheetah_amd.workloads import greedy_token
+
+    g = hip.HipForward(shape, weights(shape), quant=quant, kv_capacity=256, max_chunk_rows=32)
+    prompt = synth.make_tokens(shape.vocab_size, 20, seed=14)
+    g.forward(prompt, 0)
+    snap = g.kv_snapshot()
+
+    def at20(call, token):
+        g.clear_cache()
+        g.restore_kv_prefix(snap, 20)
+        return call(np.array([token], np.uint32), 20)
+
+    plain = at20(g.forward, 17)
+    other = at20(g.forward, 401)
+    token, logits = at20(lambda t, p: g.forward_greedy(t, p, want_logits=True), 17)
+    assert np.array_equal(bits(plain), bits(logits))
+    assert token == greedy_token(logits)
+    tail = shape.vocab_size % 4 or 4
+    assert (bits(other[-tail:]) != bits(logits[-tail:])).all()
+    token, again = at20(lambda t, p: g.forward_greedy(t, p, want_logits=True), 401)
+    assert np.array_equal(bits(other), bits(again)) and token == greedy_token(again)
+    assert np.array_equal(bits(at20(g.forward, 17)), bits(logits))
+
+
+def _attention64(q, k, v, group, offset):
+    """q [rows, heads, hd] from position offset on, k/v [ctx, kv_heads, hd]; float64."""
+    out = np.empty_like(q)
+    for r in range(q.shape[0]):
+        n = offset + r + 1
+        for h in range(q.shape[1]):
+            s = k[:n, h // group] @ q[r, h] / np.sqrt(q.shape[2])
+            w = np.exp(s - s.max())
+            out[r, h] = w @ v[:n, h // group] / w.sum()
+    return out
+
+
+@pytest.mark.parametrize("capacity", [640, 16384])
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim", [(2, 2, 64), (4, 2, 64), (7, 1, 64), (8, 1, 64), (4, 1, 128),
+                                                       (7, 1, 128)])
+def test_f32_kv_prefill_attention_holds_every_bit(hip, q_heads, kv_heads, head_dim, capacity):
+    """The f32 prefill attention alone: queries are rotated biases, K and V are
+    read back from layer 0, o_proj and layer 1's v_proj are identities, so layer
+    1's V is the RMSNorm of embedding + attention. Against 64 bits, as 2-norms:
+    two GEMM input splits (2^-18 / sqrt(3) each, 3e-6 together) and f32 scores of
+    up to 42 (2e-6 where numpy sums them in f32): 1e-5. The same with the last 8
+    bits of q, K and V cut off (the third parts left out) is 1.4e-5 to 3.4e-5 off."""
+    dim = q_heads * head_dim
+    kvd = kv_heads * head_dim
+    shape = configs.TINY_QWEN2.replace(name=f"probe-{q_heads}-{kv_heads}-{head_dim}", hidden_size=dim, q_heads=q_heads,
+                                       kv_heads=kv_heads, head_dim=head_dim)
+    w = {k: synth.bf16_to_f32(v).copy() for k, v in synth.make_weights(shape).items()}
+    p0, p1 = "model.layers.0.", "model.layers.1."
+    rng = np.random.default_rng(q_heads + head_dim)
+    scale = 8.0 / (0.02 * np.sqrt(dim))  # scores of 8 on average
+    w[p0 + "self_attn.q_proj.weight"][:] = 0
+    w[p0 + "self_attn.q_proj.bias"][:] = rng.standard_normal(dim) * scale
+    w[p0 + "self_attn.o_proj.weight"][:] = np.eye(dim)
+    w[p0 + "mlp.down_proj.weight"][:] = 0
+    w[p1 + "self_attn.v_proj.weight"][:] = np.eye(dim)[:kvd]
+    w[p1 + "self_attn.v_proj.bias"][:] = 0
+    units = {k: synth.f32_to_bf16(v) for k, v in w.items()}
+    g = hip.HipForward(shape, units, kv="f32", kv_capacity=capacity, max_chunk_rows=160)
+    n, rows = 530, 24
+    toks = synth.make_tokens(shape.vocab_size, n, seed=3)
+    g.forward(toks, 0, chunk_rows=147)
+    k, v = (t.astype(np.float64) for t in g.kv_rows(0, 0, n))
+    got = g.kv_rows(1, n - rows, rows)[1].reshape(rows, kvd)
+
+    half = head_dim // 2
+    freq = np.power(np.float32(shape.rope_theta), np.float32(-2) * np.arange(half, dtype=np.float32) / np.float32(head_dim))
+    angle = np.arange(n - rows, n, dtype=np.float32)[:, None] * freq.astype(np.float32)[None, :]
+    cos, sin = (f(angle).astype(np.float32).astype(np.float64)[:, None, :] for f in (np.cos, np.sin))
+    bias = synth.bf16_to_f32(units[p0 + "self_attn.q_proj.bias"]).astype(np.float64).reshape(1, q_heads, head_dim)
+    a, b = bias[..., :half], bias[..., half:]
+    q = np.concatenate([a * cos - b * sin, b * cos + a * sin], axis=-1).astype(np.float32).astype(np.float64)
+    embed = synth.bf16_to_f32(units["model.embed_tokens.weight"])[toks[-rows:]].astype(np.float64)
+
+    def layer1_v(q, k, v):
+        x = embed + _attention64(q, k, v, q_heads // kv_heads, n - rows).reshape(rows, dim)
+        return (x / np.sqrt((x * x).mean(axis=1, keepdims=True) + shape.rms_eps))[:, :kvd]
+
+    def cut(t):
+        return (t.astype(np.float32).view(np.uint32) & np.uint32(0xFFFFFF00)).view(np.float32).astype(np.float64)
+
+    ref = layer1_v(q, k, v)
+    off = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert off < 1e-5
+    without = np.linalg.norm(layer1_v(cut(q), cut(k), cut(v)) - ref) / np.linalg.norm(ref)
+    assert without > 1.2e-5
+
+
 @pytest.mark.parametrize("shape", TINY, ids=lambda s: s.name)
 def test_f32_kv_prefill_attention_tile_and_span_edges(hip, oracle, shape):
     """f32-cache prefill attention at the edges of its 64-key tiles, 256-key

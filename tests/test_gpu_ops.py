@@ -297,6 +297,27 @@ def test_attention_prefill_merges_more_than_64_splits(hip, hd, ctx):
         assert rel_err(got[row], ref) < 2e-5, row
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,hd", [(14, 2, 64), (16, 2, 64), (3, 1, 64), (32, 8, 128), (10, 2, 128)])
+@pytest.mark.parametrize("ctx,rows", [(37, 37), (63, 2), (64, 64), (65, 33), (127, 127), (129, 70), (1023, 65), (1025, 40),
+                                      (2113, 9)])
+def test_attention_prefill_tile_and_span_edges_with_unwritten_rows(hip, oracle, q_heads, kv_heads, hd, ctx, rows):
+    """Prefill at the edges of the 64-key tiles and the 1,024-key spans, ragged
+    row blocks, several tiles (rescaling, both buffers) and the split merge,
+    with NaN in the rows of the last page past the context: cache memory that
+    nothing has written yet, which a probability of 0 does not clear. Queries and
+    probabilities are two BF16 halves (2^-17): 2e-5 of the largest output."""
+    rng = np.random.default_rng(ctx + hd + q_heads)
+    k, v, q = _attn_case(rng, q_heads, kv_heads, hd, ctx, rows)
+    kp, vp, table = hip.paged_kv(k, v, seed=ctx)
+    if ctx % 64:
+        kp[table[-1], :, ctx % 64:] = 0x7FC0
+        vp[table[-1], :, ctx % 64:] = 0x7FC0
+    got = hip.attention(q, kp, vp, table, q_heads, rows, ctx - rows)
+    ref = oracle.attention_rows(synth.bf16_to_f32(k), synth.bf16_to_f32(v), q, q_heads, kv_heads, hd, ctx - rows)
+    assert np.isfinite(got).all()
+    assert rel_err(got, ref) < 2e-5
+
+
 def test_attention_prefill_first_calls_from_several_threads(hip, oracle):
     """The first call of a kernel lets it take its LDS, from whichever thread
     comes first: eight threads at once, each with its own buffers and scratch."""
