@@ -1047,9 +1047,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 // attention of attn_prefill_kernel (same blocks, rows per wave, LDS row
 // permutation, transposed V, delayed rescaling and split partials) with every
 // f32 operand as three BF16 parts (hi = the top 16 bits, mid = bf16 of the
-// rest, lo = what is left: all 24 bits exactly). Of the nine part products
-// the six above 2^-24 are taken, smallest first; the score's small ones add up
-// in an accumulator of their own.
+// rest, lo = what is left: all 24 bits exactly). mid is below 2^-7 of the value
+// (hi is cut, not rounded) and lo below 2^-16, so of the nine part products the
+// three left out (mid x lo twice, lo x lo) are together below 2^-22 of the
+// product; the other six are taken, smallest first, and the score's small ones
+// add up in an accumulator of their own. Their signs vary: over 128 dims the
+// scores are 6e-8 (RMS) off, f32 products summed in order 2e-7.
 //
 // Bound: the matrix cores (six BF16 products per f32 one, i.e. at most 1/6 of
 // the BF16 rate; the f32 MFMA's rate is 1/16 of it). K/V are split once per

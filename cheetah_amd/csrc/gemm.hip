@@ -476,8 +476,9 @@ template <int FMT>
 constexpr int w_row_bytes() { return FMT == FMT_BF16 ? 64 : FMT == FMT_Q8 ? 32 : 16; }
 
 // ---------------------------------------------------------------------------
-// Ring GEMM, every weight format (x pre-split, K % 32 == 0): WM x WN waves of
-// 32 MT tokens x 64 weight rows (DUAL: 32 gate and the matching 32 up rows).
+// Ring GEMM, every weight format (x pre-split; BF16 K % 32 == 0, Q8/Q4 any K on
+// halves padded with zeros): WM x WN waves of 32 MT tokens x 64 weight rows
+// (DUAL: 32 gate and the matching 32 up rows).
 // Per 32-wide K stage the block's x halves and its raw weight bytes (BF16
 // rows, Q8 codes, Q4 nibbles) go global -> LDS by buffer loads that write LDS
 // directly: a lane's source offset is fixed for the whole launch and the
@@ -497,9 +498,9 @@ constexpr int w_row_bytes() { return FMT == FMT_BF16 ? 64 : FMT == FMT_Q8 ? 32 :
 // The MFMA sequence per output and the chunk folds are those of gemm_kernel,
 // so the results are the same bits whatever the tile.
 //
-// Bound: the matrix cores, at the clock they leave (51 % busy over a wave's
-// life at 2,048 tokens x 4096 x 4096; a large BF16 product of the BLAS library
-// reaches 1.2 PFLOP/s on this card, this kernel 1.02 executed). Tiles, per
+// Bound: the matrix cores, at the clock they leave (39 to 49 % busy over a
+// dispatch of 512 tokens; a large BF16 product of the BLAS library reaches 1.2
+// PFLOP/s on this card, this kernel up to 1.08 executed). Tiles, per
 // block: 128 tokens x 256 rows on 8 waves of 64 x 64 (an LDS byte feeds 1.5
 // times the MFMAs of 32 x 64, and the block's L2 traffic per MFMA is 2/3 of
 // 128 x 128); 128 x 128 on 8 waves of 32 x 64; 64 x 128 on 4 waves, two blocks
