@@ -901,7 +901,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         for (int c = 0; c < KC; ++c) buf_to_lds<16>(rv, vs + b * TB + wave * 1024 + 4096 * c, voff, 4096 * c);
     };
     // This wave's V rows past the split end, once they have landed: they may
-    // be unwritten memory, and a probability of 0 does not clear a NaN.
+    // be unwritten memory, and a probability of 0 does not clear a NaN. (An
+    // infinite or NaN V that was written does reach the tile's earlier rows so.)
     auto clear_v = [&](int t0, int b) {
 #pragma unroll
         for (int c = 0; c < KC; ++c)
