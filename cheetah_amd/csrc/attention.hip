@@ -3,26 +3,24 @@
 // by 1/sqrt(head_dim), softmax, weighted value mix), as split-K flash
 // decoding:
 //
-//   attn_kernel (f32 K/V decode; BF16 K/V decode runs on the matrix cores,
-//   attn_dec_mfma_kernel below, and chunked prefill on attn_prefill_kernel or
-//   attn_prefill_f32_kernel): grid (splits, kv_heads, rows); block = 256
-//   threads.
-//   Each block owns one KV head, one query row and one contiguous slice of
-//   that row's visible positions [0, pos]; it streams the slice in tiles of
+//   attn_kernel (f32 K/V decode, one query row; BF16 K/V decode runs on the
+//   matrix cores, attn_dec_mfma_kernel below, and chunked prefill on
+//   attn_prefill_kernel or attn_prefill_f32_kernel): grid (splits, kv_heads);
+//   block = 256 threads.
+//   Each block owns one KV head and one contiguous slice of the row's
+//   visible positions [0, pos]; it streams the slice in tiles of
 //   64 positions (one page-aligned 64 x head_dim tile of K, then of V),
 //   scores all G = q_heads / kv_heads query heads of the group against each K
 //   row it loads (K and V are read once per group, not once per head), keeps
 //   an online softmax (running max / sum) per head and accumulates p * V.
 //   With one split it writes the normalised output; otherwise it writes a
 //   partial (unnormalised sum, max, denominator) and
-//   attn_combine_kernel merges the splits of each (row, q head) in split
-//   order, so results are deterministic.
+//   attn_combine_kernel merges the splits of each q head in split order, so
+//   results are deterministic.
 //
 // Split boundaries depend only on a row's own context length and the split
-// count. Decode is rows == 1; chunked prefill passes the chunk's rows, each
-// with its own causal length. The position base comes from a device word in
-// the decode graph (pos_dev) or from the host. K/V elements are BF16
-// (default) or f32.
+// count. The position comes from a device word in the decode graph (pos_dev)
+// or from the host. K/V elements are BF16 (default) or f32.
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -114,15 +112,14 @@ __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
     const int d8 = tid % T, pg = tid / T;
     const int split = blockIdx.x, S = gridDim.x;
     const int g = blockIdx.y;
-    const int row = blockIdx.z;
-    const long pos = (a.pos_dev ? (long)*a.pos_dev : a.offset) + row;
+    const long pos = a.pos_dev ? (long)*a.pos_dev : a.offset;
     const long ctx = pos + 1;
     long chunk = (ctx + S - 1) / S;
     chunk = (chunk + TP - 1) / TP * TP;
     const long start = (long)split * chunk;
     const long end = min(start + chunk, ctx);
     const size_t part_head = (size_t)S * (HD + 2);
-    float *part = a.part + ((size_t)row * a.q_heads + (size_t)g * G) * part_head + (size_t)split * (HD + 2);
+    float *part = a.part + (size_t)g * G * part_head + (size_t)split * (HD + 2);
 
     if (start >= ctx) {  // empty split: contributes nothing to the merge
         if (tid < G) part[tid * part_head + HD] = -INFINITY;
@@ -133,7 +130,7 @@ __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
     float qr[G][8];
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-        const float *qp = a.q + (size_t)row * a.q_stride + (size_t)(g * G + j) * HD + d8 * 8;
+        const float *qp = a.q + (size_t)(g * G + j) * HD + d8 * 8;
         const f32x4 q0 = *(const f32x4 *)qp, q1 = *(const f32x4 *)(qp + 4);
         qr[j][0] = q0[0]; qr[j][1] = q0[1]; qr[j][2] = q0[2]; qr[j][3] = q0[3];
         qr[j][4] = q1[0]; qr[j][5] = q1[1]; qr[j][6] = q1[2]; qr[j][7] = q1[3];
@@ -285,14 +282,14 @@ __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
     for (int t = tid; t < G * HD; t += kThreads) {
         const int j = t / HD, d = t % HD;
         const float o = s_red[0][j][d] + s_red[1][j][d] + s_red[2][j][d] + s_red[3][j][d];
-        if constexpr (DIRECT) a.out[((size_t)row * a.q_heads + g * G + j) * HD + d] = o / s_l[j];
+        if constexpr (DIRECT) a.out[(size_t)(g * G + j) * HD + d] = o / s_l[j];
         else part[j * part_head + d] = o;
     }
 }
 
 // ---------------------------------------------------------------------------
 // Decode attention on the matrix cores (BF16 KV, head_dim 64 or 128, up to 8
-// query heads per KV head): grid (splits, kv_heads, rows) as attn_kernel, the
+// query heads per KV head): grid (splits, kv_heads) as attn_kernel, the
 // same split boundaries and partial layout. The block's positions are cut
 // into 32-position tiles dealt round-robin to its 4 waves; each wave runs its
 // own online softmax over its tiles with no block barrier, and the 4 wave
@@ -348,15 +345,14 @@ __global__ __launch_bounds__(kThreads) void attn_dec_mfma_kernel(AttnArgs a) {
     const int n = lane & 15, kg = lane >> 4;
     const int split = blockIdx.x, S = gridDim.x;
     const int g = blockIdx.y;
-    const int row = blockIdx.z;
-    const long pos = (a.pos_dev ? (long)*a.pos_dev : a.offset) + row;
+    const long pos = a.pos_dev ? (long)*a.pos_dev : a.offset;
     const long ctx = pos + 1;
     long chunk = (ctx + S - 1) / S;
     chunk = (chunk + TP - 1) / TP * TP;
     const long start = (long)split * chunk;
     const long end = min(start + chunk, ctx);
     const size_t part_head = (size_t)S * (HD + 2);
-    float *part = a.part + ((size_t)row * a.q_heads + (size_t)g * G) * part_head + (size_t)split * (HD + 2);
+    float *part = a.part + (size_t)g * G * part_head + (size_t)split * (HD + 2);
     if (start >= ctx) {  // empty split: contributes nothing to the merge
         if (threadIdx.x < G) part[threadIdx.x * part_head + HD] = -INFINITY;
         return;
@@ -369,7 +365,7 @@ __global__ __launch_bounds__(kThreads) void attn_dec_mfma_kernel(AttnArgs a) {
     // tile registers (bits equal to what the cache will hold).
     __shared__ __attribute__((aligned(16))) uint16_t s_new[2][HD];
     const int q_dim = a.q_heads * HD, kv_dim = a.kv_heads * HD, half = a.rotary_dim / 2;
-    const float *qkv_row = ROPE ? a.qkv + (size_t)row * (q_dim + 2 * kv_dim) : nullptr;
+    const float *qkv_row = ROPE ? a.qkv : nullptr;
     const float *cr = ROPE ? a.rope_cos + (size_t)pos * half : nullptr;
     const float *sr = ROPE ? a.rope_sin + (size_t)pos * half : nullptr;
     const int pos_tile = (int)((pos - start) / TW);  // tile index of pos in this block's range
@@ -552,7 +548,7 @@ __global__ __launch_bounds__(kThreads) void attn_dec_mfma_kernel(AttnArgs a) {
                 qcs[s][2] = *(const f32x4 *)(sr + i0);
                 qcs[s][3] = *(const f32x4 *)(sr + i0 + 4);
             } else {
-                const float *qp = a.q + (size_t)row * a.q_stride + (size_t)(g * G + (n < G ? n : 0)) * HD + 32 * s + 8 * kg;
+                const float *qp = a.q + (size_t)(g * G + (n < G ? n : 0)) * HD + 32 * s + 8 * kg;
                 qraw[s][0] = *(const f32x4 *)qp;
                 qraw[s][1] = *(const f32x4 *)(qp + 4);
             }
@@ -624,7 +620,7 @@ __global__ __launch_bounds__(kThreads) void attn_dec_mfma_kernel(AttnArgs a) {
             }
         }
         if constexpr (DIRECT) {
-            a.out[((size_t)row * a.q_heads + g * G + j) * HD + d] = acc / L;
+            a.out[(size_t)(g * G + j) * HD + d] = acc / L;
         } else {
             part[j * part_head + d] = acc;
             if (d == 0) {
@@ -635,17 +631,17 @@ __global__ __launch_bounds__(kThreads) void attn_dec_mfma_kernel(AttnArgs a) {
     }
 }
 
-// Merge the splits of one (row, q head) in split order: one wave turns the
+// Merge the splits of one q head in split order: one wave turns the
 // split maxima into weights w_s = exp(m_s - M) and 1 / sum_s w_s l_s, then
 // all threads sum w_s * o_s[d] over the non-empty splits.
 template <int HD>
-__global__ __launch_bounds__(kThreads) void attn_combine_kernel(const float *part, int S, int q_heads, float *out) {
+__global__ __launch_bounds__(kThreads) void attn_combine_kernel(const float *part, int S, float *out) {
     constexpr int GR = kThreads / HD;  // split groups
     __shared__ float s_w[kMaxSplits];
     __shared__ float s_inv;
     __shared__ float s_o[GR][HD];
-    const int h = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
-    const float *p = part + ((size_t)row * q_heads + h) * (size_t)S * (HD + 2);
+    const int h = blockIdx.x, tid = threadIdx.x;
+    const float *p = part + (size_t)h * (size_t)S * (HD + 2);
     static_assert(kMaxSplits <= 128, "one wave holds two splits per lane");
     if (tid < 64) {
         const int s1 = tid + 64;
@@ -687,7 +683,7 @@ __global__ __launch_bounds__(kThreads) void attn_combine_kernel(const float *par
         float sum = s_o[0][tid];
 #pragma unroll
         for (int k = 1; k < GR; ++k) sum += s_o[k][tid];
-        out[((size_t)row * q_heads + h) * HD + tid] = sum * s_inv;
+        out[(size_t)h * HD + tid] = sum * s_inv;
     }
 }
 
@@ -1681,7 +1677,7 @@ int launch_prefill_h(const AttnJob &j, const AttnArgs &a, int G, int S, hipStrea
 // ALUs.
 template <int HD, int G, class KT>
 int launch_hgk(const AttnJob &j, const AttnArgs &a, hipStream_t s) {
-    const dim3 grid(j.splits, j.g.kv_heads, j.rows);
+    const dim3 grid(j.splits, j.g.kv_heads);
     constexpr bool mfma = std::is_same<KT, uint16_t>::value;
     const bool rope = a.qkv != nullptr;
     if (rope && !mfma) return fail("HIP backend: fused RoPE needs the matrix-core attention kernel.");
@@ -1702,8 +1698,7 @@ int launch_hgk(const AttnJob &j, const AttnArgs &a, hipStream_t s) {
         hipLaunchKernelGGL((attn_kernel<HD, G, KT, false>), grid, dim3(kThreads), 0, s, a);
     }
     CHIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL((attn_combine_kernel<HD>), dim3(j.q_heads, j.rows), dim3(kThreads), 0, s, a.part, j.splits,
-                       j.q_heads, a.out);
+    hipLaunchKernelGGL((attn_combine_kernel<HD>), dim3(j.q_heads), dim3(kThreads), 0, s, a.part, j.splits, a.out);
     CHIP_CHECK(hipGetLastError());
     return 0;
 }
@@ -1780,14 +1775,9 @@ bool attention_decode_fuses_rope(const KvGeom &g, int q_heads, int rotary_dim) {
            q_heads % g.kv_heads == 0 && q_heads / g.kv_heads <= 8 && rotary_dim == g.head_dim;
 }
 
-bool attention_prefill_on_mfma(const KvGeom &g, int q_heads) {
-    return (g.head_dim == 64 || g.head_dim == 128) && g.kv_heads > 0 && q_heads % g.kv_heads == 0 &&
-           q_heads / g.kv_heads <= 8;
-}
-
 int launch_attention(const AttnJob &j, hipStream_t s) {
     if (j.rows == 0) return 0;
-    const bool halves_only = j.prefill && j.out_hi && attention_prefill_on_mfma(j.g, j.q_heads);
+    const bool halves_only = j.prefill && j.out_hi;
     if ((!j.q && !j.qkv) || (!j.out && !halves_only) || !j.k || !j.v || !j.g.page_table || (!j.prefill && j.splits > 1 && !j.part))
         return fail("HIP backend: attention is missing a buffer.");
     if (j.g.kv_heads <= 0 || j.q_heads <= 0 || j.q_heads % j.g.kv_heads)
@@ -1819,7 +1809,10 @@ int launch_attention(const AttnJob &j, hipStream_t s) {
         a.rotary_dim = j.rotary_dim;
     }
     const int G = j.q_heads / j.g.kv_heads;
-    if (j.prefill && attention_prefill_on_mfma(j.g, j.q_heads)) {
+    if (j.g.head_dim != 64 && j.g.head_dim != 128) return fail("HIP backend: attention supports head_dim 64 and 128.");
+    if (G > 8) return fail("HIP backend: attention supports 1..8 query heads per KV head.");
+    if (!j.prefill && j.rows != 1) return fail("HIP backend: decode attention takes one row.");
+    if (j.prefill) {
         if (j.pos_dev) return fail("HIP backend: prefill attention takes a host position.");
         if (j.offset + j.rows > (size_t)INT32_MAX) return fail("HIP backend: prefill position out of range.");
         if (j.span < 64 || j.span % 64) return fail("HIP backend: prefill span must be a positive multiple of 64.");
@@ -1835,8 +1828,7 @@ int launch_attention(const AttnJob &j, hipStream_t s) {
         return launch_prefill_h<128>(j, a, G, S, s);
     }
     if (j.g.head_dim == 64) return launch_h<64>(j, a, G, s);
-    if (j.g.head_dim == 128) return launch_h<128>(j, a, G, s);
-    return fail("HIP backend: attention supports head_dim 64 and 128.");
+    return launch_h<128>(j, a, G, s);
 }
 
 }  // namespace chip

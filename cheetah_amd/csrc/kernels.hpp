@@ -168,8 +168,9 @@ int launch_gather_rows(const uint8_t *src, uint8_t *dst, const int32_t *map, siz
                        hipStream_t s);
 
 // GQA attention for `rows` query rows at positions pos0 + i over keys
-// [0, pos0 + i]. q row stride q_stride floats. The split count (at most
-// attention_max_splits()) is the caller's: decode graphs need a fixed grid.
+// [0, pos0 + i]; head_dim 64 or 128, at most 8 query heads per KV head. q row
+// stride q_stride floats. Without `prefill` one row, and the split count (at
+// most attention_max_splits()) is the caller's: decode graphs need a fixed grid.
 // Partial buffers hold rows * q_heads * splits * (head_dim + 2) floats.
 // Keys per split of the matrix-core chunked prefill when the caller names
 // no span (attention_prefill_span gives a model's).
@@ -189,9 +190,8 @@ struct AttnJob {
     const int32_t *pos_dev = nullptr;
     int splits = 1;
     float *part = nullptr;  // partial buffer (splits > 1)
-    // Chunked prefill (host offset): head_dim 64/128 runs on the
-    // matrix cores with attention_prefill_splits(offset + rows) splits and
-    // ignores `splits`; part must then hold part_floats >= the partials.
+    // Chunked prefill (host offset): attention_prefill_splits(offset + rows)
+    // splits, `splits` ignored; part must then hold part_floats >= the partials.
     bool prefill = false;
     size_t part_floats = 0;
     // Keys per prefill split (absolute position ranges [s span, (s+1) span)):
@@ -204,10 +204,9 @@ struct AttnJob {
     const float *qkv = nullptr;
     const float *rope_cos = nullptr, *rope_sin = nullptr;
     int rotary_dim = 0;
-    // Chunked prefill on the matrix cores (attention_prefill_on_mfma) also
-    // writes out's BF16 halves here when set: hi = bf16(v), lo = bf16(v - hi),
-    // the bits launch_split_bf16 would write; out may then be null. Other
-    // paths ignore them.
+    // Chunked prefill also writes out's BF16 halves here when set: hi =
+    // bf16(v), lo = bf16(v - hi), the bits launch_split_bf16 would write; out
+    // may then be null. Decode ignores them.
     uint16_t *out_hi = nullptr, *out_lo = nullptr;
 };
 int launch_attention(const AttnJob &job, hipStream_t s);
@@ -225,7 +224,6 @@ int attention_prefill_splits(size_t ctx, int span = kDefaultPrefillSpan);
 // most capacity / 8, and at least kDefaultPrefillSpan (f32 cache:
 // kF32PrefillSpan).
 int attention_prefill_span(size_t kv_capacity, bool kv_f32);
-bool attention_prefill_on_mfma(const KvGeom &g, int q_heads);
 
 // Greedy argmax (ties -> last index, total order) of logits[n]; writes the
 // index to *out_token. When `step` is set (the device-side decode loop,
