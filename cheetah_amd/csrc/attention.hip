@@ -1121,7 +1121,8 @@ constexpr float kBigV = 0x1p119f;
 // One row's attention over positions [p0, p1) in plain f32 products, parts of
 // `sub` positions folded in order, a lane's HD / 2 dims of it stored as
 // store_prefill_rows does: the rare rows whose operands the BF16 parts do not
-// carry. A call, so that it takes no registers of the loop's.
+// carry. A call, so that it takes no registers of the loop's. A NaN weight sum
+// is the row's result: it ends there, with a maximum that no split outweighs.
 template <int HD>
 __device__ __attribute__((noinline)) void plain_row(AttnArgs a, int row, int head, int g, int half, int p0, int p1, int sub,
                                               float *part, int S) {
@@ -1133,13 +1134,13 @@ __device__ __attribute__((noinline)) void plain_row(AttnArgs a, int row, int hea
 #pragma unroll
     for (int u = 0; u < UT; ++u) o[u] = f32x16{};
 #pragma unroll 1
-    for (; p0 < p1; p0 += sub) {
+    for (; p0 < p1 && L == L; p0 += sub) {
         f32x16 t[UT];
         float m = -INFINITY, l = 0.f;
 #pragma unroll
         for (int u = 0; u < UT; ++u) t[u] = f32x16{};
 #pragma unroll 1
-        for (int p = p0; p < min(p0 + sub, p1); ++p) {
+        for (int p = p0; p < min(p0 + sub, p1) && l == l; ++p) {
             const size_t at = (((size_t)a.page_table[p / a.page_size] * a.kv_heads + g) * a.page_size + p % a.page_size) * HD;
             const float *kp = (const float *)a.k + at, *vp = (const float *)a.v + at + 4 * half;
             float dot = 0.f;
@@ -1168,6 +1169,7 @@ __device__ __attribute__((noinline)) void plain_row(AttnArgs a, int row, int hea
                 }
         }
         float alpha, beta;
+        if (l != l) m = INFINITY;
         const bool any = m != -INFINITY;
         fold_factors(m, M, alpha, beta);
         L = any ? fold_value(L, l, alpha, beta) : L;

@@ -303,6 +303,32 @@ def test_f32_kv_infinite_value_reaches_no_earlier_row(hip, head_dim, capacity):
 
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("capacity", [640, 16384])
+def test_f32_kv_nan_key_reaches_every_later_row_and_no_earlier_one(hip, head_dim, capacity):
+    """Layer 0 gives token 7 NaN keys (an infinity through the rotation): every
+    row from it on is NaN, whatever split the key is in, and the rows before it
+    keep their bits."""
+    def edit(w, shape):
+        w["model.layers.0.self_attn.k_proj.weight"][:, 5] = 3e38 * np.where(np.arange(shape.kv_dim) % 2, 1, -1)
+
+    shape, w = _marked_model(head_dim, edit)
+    g = hip.HipForward(shape, w, kv="f32", kv_capacity=capacity, max_chunk_rows=160)
+    toks = synth.make_tokens(shape.vocab_size, 600, seed=15)
+    toks[toks == 7] = 8
+    g.forward(toks, 0, chunk_rows=160)
+    want = g.kv_rows(1, 0, 600)
+    for at in (5, 300):
+        g.clear_cache()
+        both = toks.copy()
+        both[at] = 7
+        assert np.isnan(g.forward(both, 0, chunk_rows=160)).all()
+        assert np.isnan(g.kv_rows(0, at, 1)[0]).any()
+        for x, y in zip(g.kv_rows(1, 0, 600), want):
+            assert np.array_equal(bits(x[:at]), bits(y[:at]))
+            assert np.isnan(x[at:]).all()
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("capacity", [640, 16384])
 def test_f32_kv_score_of_minus_infinity_weighs_nothing(hip, oracle, head_dim, capacity):
     """Token 7's keys and every query hold large values of opposite signs in the
     slowest rotary pair: their product is past the largest f32, -inf, and
